@@ -268,6 +268,54 @@ hipError_t launch_attention(hipStream_t s, const AttnArgs &a, int head_dim, int 
 hipError_t launch_embed(hipStream_t s, const EmbedArgs &a, int batch);
 // fp16 out16[b] = norm(x[b]) (pro = kProRms or kProLayer), K <= 4096.
 hipError_t launch_norm_rows(hipStream_t s, const GemvArgs &a, int pro);
+
+// ---- prompts in one pass (prefill.hip) -------------------------------------------
+
+// C = A W^T over M token rows: A fp16 [M][lda], W tiled (N % 64 == 0, K % 128
+// == 0), scales and biases as the GEMV's; epilogues kEpiStore, kEpiResidual
+// (out += ), kEpiSwiGLU (FP8) and kEpiGelu (fp16).
+struct PrefillGemmArgs {
+  const uint8_t *w = nullptr;
+  const float *scale = nullptr, *bias = nullptr;
+  const uint16_t *a = nullptr;
+  int lda = 0, M = 0, K = 0, N = 0;
+  float *out = nullptr;
+  uint16_t *out16 = nullptr;
+  int out_ld = 0;
+};
+
+// A chunk of a prompt: tokens i0 .. i0 + T - 1 of B sequences, token row
+// m = b * T + i at position lens[b] + i0 + i; then one layer's q / k / v.
+struct PrefillArgs {
+  const int *tokens = nullptr;  // [B][prompt_len]
+  const int *lens = nullptr;    // [B] positions cached before the prompt
+  int prompt_len = 0, i0 = 0, T = 0, B = 0;
+  int H = 0, heads = 0, kv_heads = 0, d = 0, qkv_n = 0, max_pos = 0;
+  int vt_stride = 0;            // positions per V^T cache row; 0: V as [max_pos][d]
+  float eps = 0.0f, scale = 1.0f;
+  // embedding
+  int *hist = nullptr;
+  int hist_len = 0;
+  const uint8_t *head8 = nullptr;
+  const float *head_scale = nullptr;
+  const uint16_t *head16 = nullptr, *wpe = nullptr;
+  const float *inv_freq = nullptr;
+  float *rope = nullptr;        // [B * T][d]: cos | sin
+  float *x = nullptr;           // [B * T][H] residual stream
+  // attention
+  const float *qkv = nullptr, *q_norm = nullptr, *k_norm = nullptr;  // qkv [B * T][qkv_n]
+  uint16_t *q = nullptr, *q_lo = nullptr;  // [B * T][heads][d], scaled
+  uint16_t *kcache = nullptr, *vcache = nullptr;
+  uint16_t *attn = nullptr;     // [B * T][heads * d] fp16
+};
+hipError_t launch_prefill_embed(hipStream_t s, const PrefillArgs &a);
+hipError_t launch_prefill_gemm(hipStream_t s, const PrefillGemmArgs &g, int weight_type, int epi);
+// q, k, v of a layer: norms and RoPE, q out, k and v appended to the caches
+// (kv_only: without the query heads).
+hipError_t launch_prefill_qkv(hipStream_t s, const PrefillArgs &a, bool qwen, bool kv_only);
+hipError_t launch_prefill_attention(hipStream_t s, const PrefillArgs &a);
+hipError_t launch_prefill_finish(hipStream_t s, int *lens, int B, int n);  // lens[b] += n
+
 hipError_t launch_quantize_e4m3_tiled(hipStream_t s, const float *w, int N, int K,
                                       int interleave_rows, uint8_t *q, float *scales,
                                       bool tiled);
