@@ -92,7 +92,7 @@ __global__ void prefill_finish_kernel(int *lens, int B, int n) {
 // issued as W x A, which leaves a lane with 4 consecutive outputs of one
 // token (16-byte fp32, 8-byte fp16 stores).
 template <int kW, int kEpi, int kMI>
-__global__ __launch_bounds__(kT) void prefill_gemm_kernel(const PrefillGemmArgs g, int tiles_m,
+__global__ __launch_bounds__(kT, kMI == 4 ? 2 : 4) void prefill_gemm_kernel(const PrefillGemmArgs g, int tiles_m,
                                                           int ntiles, int per_xcd) {
   constexpr int kBM = 32 * kMI;
   constexpr int kChunks = kBM * 8 / kT;            // 16-byte chunks per thread and stage
@@ -177,14 +177,20 @@ __global__ __launch_bounds__(kT) void prefill_gemm_kernel(const PrefillGemmArgs 
   // barrier that ended the previous stage)
   for (int kt = 0; kt < nk; kt += 2) {
     const int k2 = min(kt + 2, nk - 1), k3 = min(kt + 3, nk - 1);  // past the end: re-read, unused
+    // (the order is kept: a store moved up ahead of the loads would wait for
+    // the stage requested last, not the one before it)
     load_a(0, k2);
+    __builtin_amdgcn_sched_barrier(0);
     compute(0, 0);
     load_w(0, k2);
+    __builtin_amdgcn_sched_barrier(0);
     store_a(1, 1);
     lds_barrier();
     load_a(1, k3);
+    __builtin_amdgcn_sched_barrier(0);
     compute(1, 1);
     load_w(1, k3);
+    __builtin_amdgcn_sched_barrier(0);
     store_a(0, 0);
     lds_barrier();
   }
