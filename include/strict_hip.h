@@ -370,8 +370,9 @@ SH_API int sh_rgb_to_bgr_u8(sh_ctx *ctx, const uint8_t *src, uint8_t *dst, int w
 /* C[M,N] = A[M,K] * B[K,N]: bf16 operands (raw 16-bit patterns), fp32
  * accumulation, bf16 result (round to nearest even), row-major with leading
  * dimensions lda >= K, ldb >= N, ldc >= N (elements). K == 0 writes zeros.
- * The MFMA path needs M, N multiples of 256, K of 64, lda/ldb multiples of 8
- * and 16-byte aligned A/B; other shapes run a slower exact-fp32 kernel. */
+ * Every shape and alignment runs on MFMA; the fastest kernel takes over 128
+ * tiles of 256 x 256 with K a multiple of 32, lda / ldb of 8, ldc of 4 and
+ * 16-byte aligned A / B. */
 SH_API int sh_gemm_bf16(sh_ctx *ctx, const uint16_t *A, const uint16_t *B, uint16_t *C, int M,
                         int N, int K, int lda, int ldb, int ldc);
 
@@ -380,10 +381,10 @@ SH_API int sh_gemm_bf16(sh_ctx *ctx, const uint16_t *A, const uint16_t *B, uint1
  * row-major [M][K] (lda >= K bytes), B arrives transposed as Bt [N][K]
  * (ldb >= K bytes; a weight matrix W[N][K]), C row-major (ldc >= N
  * elements); sa (M floats) and sb (N floats) are the per-row / per-column
- * scales sh_quantize_e4m3 produces. K == 0 writes zeros. The MFMA path needs
- * M, N multiples of 256, K of 128, lda / ldb multiples of 16, 16-byte aligned
- * A, Bt and sb; other shapes run a slower exact-fp32 kernel. No counterpart in
- * the reference (BASELINE's FP8 GEMM measurement). */
+ * scales sh_quantize_e4m3 produces. K == 0 writes zeros. Every shape and
+ * alignment runs on MFMA; the fastest kernel takes over 96 tiles of 256 x 256
+ * with K a multiple of 128, lda / ldb of 16, ldc of 4 and 16-byte aligned A,
+ * Bt and sb. No counterpart in the reference. */
 SH_API int sh_gemm_fp8(sh_ctx *ctx, const uint8_t *A, const float *sa, const uint8_t *Bt,
                        const float *sb, uint16_t *C, int M, int N, int K, int lda, int ldb,
                        int ldc);

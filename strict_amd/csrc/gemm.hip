@@ -20,12 +20,14 @@
 //  - tiles are numbered so that each of the 8 XCDs (workgroups are dealt to
 //    XCDs round-robin) computes a 4 x 8 block of tiles, whose A and B slabs
 //    its L2 then shares.
-// Every other shape takes a bounds-checked LDS-tiled fp32 FMA kernel.
+// Every other shape, and one of too few such tiles, takes the kernel of
+// gemm_edge.h.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
 
 #include "common.h"
+#include "gemm_edge.h"
 
 namespace sh {
 namespace {
@@ -270,59 +272,6 @@ void gemm_bf16_mfma_kernel(const uint16_t *__restrict__ A, const uint16_t *__res
   }
 }
 
-// ---- generic path: any shape and leading dimensions ----------------------
-
-constexpr int kGT = 64;  // 64 x 64 tile, 256 threads, 4 x 4 outputs each
-
-__device__ __forceinline__ float bf16_bits_to_f32(uint16_t h) {
-  return __builtin_bit_cast(float, (uint32_t)h << 16);
-}
-
-__global__ __launch_bounds__(256) void gemm_bf16_generic_kernel(const uint16_t *A,
-                                                                const uint16_t *B, uint16_t *C,
-                                                                int M, int N, int K, int lda,
-                                                                int ldb, int ldc) {
-  __shared__ float as[16][kGT + 1];
-  __shared__ float bs[16][kGT + 1];
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const int m0 = blockIdx.y * kGT, n0 = blockIdx.x * kGT;
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    for (int idx = threadIdx.x; idx < 16 * kGT; idx += 256) {
-      const int kk = idx & 15, mm = idx >> 4;  // A tile: 64 rows x 16 k
-      const int gm = m0 + mm, gk = k0 + kk;
-      as[kk][mm] = (gm < M && gk < K) ? bf16_bits_to_f32(A[(size_t)gm * lda + gk]) : 0.0f;
-      const int nn = idx & 63, kb = idx >> 6;  // B tile: 16 k x 64 cols
-      const int gn = n0 + nn, gk2 = k0 + kb;
-      bs[kb][nn] = (gn < N && gk2 < K) ? bf16_bits_to_f32(B[(size_t)gk2 * ldb + gn]) : 0.0f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < 16; kk++) {
-      float a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; i++) a[i] = as[kk][ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; j++) b[j] = bs[kk][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int gm = m0 + ty * 4 + i;
-    if (gm >= M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int gn = n0 + tx * 4 + j;
-      if (gn < N) C[(size_t)gm * ldc + gn] = (uint16_t)f32_to_bf16_bits(acc[i][j]);
-    }
-  }
-}
-
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 }  // namespace
@@ -332,7 +281,11 @@ bool gemm_bf16_uses_mfma(int M, int N, int K, int lda, int ldb, int ldc, const v
   return M % kBM == 0 && N % kBN == 0 && K % kDK == 0 && K > 0 && lda % 8 == 0 &&
          ldb % 8 == 0 && ldc % 4 == 0 && aligned16(A) && aligned16(B) &&
          (reinterpret_cast<uintptr_t>(C) & 7) == 0 && (int64_t)kBM * lda * 2 < (1ll << 31) &&
-         (int64_t)K * ldb * 2 < (1ll << 31);
+         (int64_t)K * ldb * 2 < (1ll << 31) &&
+         // more than half of the CUs have a tile: 4096 x 2048 x 1024 (128 tiles)
+         // took 33.1 us against 29.3 with 128 x 128 tiles, 2048^3 (64) 45.7
+         // against 32.4, but 3072^3 (144) 65.1 against 92.4
+         (int64_t)(M / kBM) * (N / kBN) > 128;
 }
 
 hipError_t launch_gemm_bf16(hipStream_t s, const uint16_t *A, const uint16_t *B, uint16_t *C,
@@ -350,8 +303,19 @@ hipError_t launch_gemm_bf16(hipStream_t s, const uint16_t *A, const uint16_t *B,
     e = hipLaunchKernel(kfn, dim3(ntiles), dim3(kThreads), args, lds_bytes, s);
     if (e != hipSuccess) return e;
   } else {
-    dim3 grid((N + kGT - 1) / kGT, (M + kGT - 1) / kGT);
-    gemm_bf16_generic_kernel<<<grid, 256, 0, s>>>(A, B, C, M, N, K, lda, ldb, ldc);
+    edge::Args g = {};
+    g.a = reinterpret_cast<const uint8_t *>(A);
+    g.b = reinterpret_cast<const uint8_t *>(B);
+    g.c = C;
+    g.M = M;
+    g.N = N;
+    g.K = K;
+    g.lda = (size_t)lda * 2;
+    g.ldb = (size_t)ldb * 2;
+    g.ldc = ldc;
+    g.span_a = ((size_t)(M - 1) * lda + K) * 2;
+    g.span_b = ((size_t)(K - 1) * ldb + N) * 2;
+    return edge::launch<false>(s, g);
   }
   return hipGetLastError();
 }

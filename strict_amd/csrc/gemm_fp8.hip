@@ -30,17 +30,18 @@
 //  - issued as Bt x A so that each lane holds one row of C with runs of four
 //    consecutive columns;
 //  - XCD-grouped tile order as in the bf16 kernel.
-// Every other shape takes a bounds-checked fp32 FMA kernel.
+// Every other shape, and one of too few such tiles, takes the kernel of
+// gemm_edge.h.
 #include <hip/hip_runtime.h>
 
 #include "common.h"
+#include "gemm_edge.h"
 
 namespace sh {
 namespace {
 
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kBM = 256, kBN = 256, kBK = 128;  // kBK in bytes = fp8 values
 constexpr int kThreads = 256;
@@ -230,59 +231,6 @@ void gemm_fp8_mfma_kernel(const uint8_t *__restrict__ A, const float *__restrict
   }
 }
 
-// ---- generic path: any shape and leading dimensions ----------------------
-
-constexpr int kGT = 64;  // 64 x 64 tile, 256 threads, 4 x 4 outputs each
-
-__device__ __forceinline__ float e4m3_to_f32(uint8_t q) {
-  const f16x2 h = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((uint32_t)q, 1.0f, false);
-  return (float)h[0];
-}
-
-__global__ __launch_bounds__(256) void gemm_fp8_generic_kernel(const uint8_t *A, const float *sa,
-                                                               const uint8_t *Bt, const float *sb,
-                                                               uint16_t *C, int M, int N, int K,
-                                                               int lda, int ldb, int ldc) {
-  __shared__ float as[16][kGT + 1];
-  __shared__ float bs[16][kGT + 1];
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const int m0 = blockIdx.y * kGT, n0 = blockIdx.x * kGT;
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    for (int idx = threadIdx.x; idx < 16 * kGT; idx += 256) {
-      const int kk = idx & 15, rr = idx >> 4;  // 64 rows x 16 k of each operand
-      const int gk = k0 + kk;
-      const int gm = m0 + rr, gn = n0 + rr;
-      as[kk][rr] = (gm < M && gk < K) ? e4m3_to_f32(A[(size_t)gm * lda + gk]) : 0.0f;
-      bs[kk][rr] = (gn < N && gk < K) ? e4m3_to_f32(Bt[(size_t)gn * ldb + gk]) : 0.0f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < 16; kk++) {
-      float a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; i++) a[i] = as[kk][ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; j++) b[j] = bs[kk][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int gm = m0 + ty * 4 + i;
-    if (gm >= M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int gn = n0 + tx * 4 + j;
-      if (gn < N) C[(size_t)gm * ldc + gn] = (uint16_t)f32_to_bf16_bits(acc[i][j] * sa[gm] * sb[gn]);
-    }
-  }
-}
-
 bool aligned(const void *p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
 }  // namespace
@@ -291,7 +239,11 @@ bool gemm_fp8_uses_mfma(int M, int N, int K, int lda, int ldb, int ldc, const vo
                         const void *Bt, const void *C, const void *sb) {
   return M % kBM == 0 && N % kBN == 0 && K % kBK == 0 && K > 0 && lda % 16 == 0 &&
          ldb % 16 == 0 && ldc % 4 == 0 && aligned(A, 16) && aligned(Bt, 16) && aligned(C, 8) &&
-         aligned(sb, 16) && (int64_t)kBM * lda < (1ll << 31) && (int64_t)kBN * ldb < (1ll << 31);
+         aligned(sb, 16) && (int64_t)kBM * lda < (1ll << 31) && (int64_t)kBN * ldb < (1ll << 31) &&
+         // over a third of the CUs have a tile: 2560 x 2048 x 1024 (80 tiles)
+         // took 26.3 us against the other kernel's 19.1, 2048^3 (64) 34.5 against
+         // 27.8, but 2304 x 2816 x 2048 (99) 35.0 against 39.4
+         (int64_t)(M / kBM) * (N / kBN) > 96;
 }
 
 hipError_t launch_gemm_fp8(hipStream_t s, const uint8_t *A, const float *sa, const uint8_t *Bt,
@@ -307,8 +259,21 @@ hipError_t launch_gemm_fp8(hipStream_t s, const uint8_t *A, const float *sa, con
     gemm_fp8_mfma_kernel<<<ntiles, kThreads, kLdsBytes, s>>>(A, sa, Bt, sb, C, K, lda, ldb, ldc,
                                                             tiles_m, tiles_n, grouped);
   } else {
-    dim3 grid((N + kGT - 1) / kGT, (M + kGT - 1) / kGT);
-    gemm_fp8_generic_kernel<<<grid, 256, 0, s>>>(A, sa, Bt, sb, C, M, N, K, lda, ldb, ldc);
+    edge::Args g = {};
+    g.a = A;
+    g.b = Bt;
+    g.sa = sa;
+    g.sb = sb;
+    g.c = C;
+    g.M = M;
+    g.N = N;
+    g.K = K;
+    g.lda = (size_t)lda;
+    g.ldb = (size_t)ldb;
+    g.ldc = ldc;
+    g.span_a = (size_t)(M - 1) * lda + K;
+    g.span_b = (size_t)(N - 1) * ldb + K;
+    return edge::launch<true>(s, g);
   }
   return hipGetLastError();
 }
