@@ -18,6 +18,9 @@
 // products x * q are exact and the scale is applied once to the fp32 sum.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "common.h"
 #include "llm.h"
 #include "llm_device.h"
@@ -394,6 +397,69 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(const GemvArgs a) {
           k > __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
         atomicMax(slot, k);
     }
+  }
+}
+
+// ---- GEMV with the activations in registers ---------------------------------
+
+// y[b][n] = scale[n] * sum_k x[b][k] W[n][k] for K = 256 kL: the store-only FP8
+// GEMV of gemv_kernel, same sums in the same order, without its LDS copy of
+// the activations. Each of the 4 waves holds its quarter of K of all 16 rows
+// as MFMA operands (8 kL registers), so nothing but the weights streams in the
+// loop and LDS only carries the 4 partial tiles. A workgroup goes over its
+// 16-row tiles with the next tile's weights requested before a tile's MFMAs
+// and one barrier per tile (the partials alternate between two buffers; a
+// wave adds and stores a quarter of the tile's rows).
+template <int kL>
+__global__ __launch_bounds__(kThreads, kL <= 4 ? 4 : 2) void gemv_regs_kernel(const GemvArgs a) {
+  __shared__ f32x4 red[2][4][64];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int col = lane & 15, grp = lane >> 4;
+  const int tiles = a.N / 16;
+  f16x8 af[2 * kL];
+#pragma unroll
+  for (int i = 0; i < 2 * kL; i++) {
+    // (rows past the batch read its last row: their sums are not stored)
+    af[i] = *reinterpret_cast<const f16x8 *>(a.act + (size_t)min(col, a.B - 1) * a.act_ld +
+                                             wave * (kL * 64) + 32 * i + 8 * grp);
+  }
+  const uint8_t *w = a.w + (size_t)wave * kL * 1024 + (size_t)lane * 16;
+  u32x4 wv[2][kL];
+  auto load = [&](int s, int g) __attribute__((always_inline)) {
+    const uint8_t *p = w + (size_t)min(g, tiles - 1) * (kL * 4 * 1024);
+#pragma unroll
+    for (int u = 0; u < kL; u++)
+      wv[s][u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p + u * 1024));
+  };
+  auto step = [&](int g, auto par_c) __attribute__((always_inline)) {
+    constexpr int kPar = decltype(par_c)::value;
+    const float sc = a.scale[g * 16 + col];
+    load(kPar ^ 1, g + gridDim.x);
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < kL; u++)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+            af[2 * u + h], e4m3x8_to_f16(wv[kPar][u][2 * h], wv[kPar][u][2 * h + 1]), acc, 0, 0, 0);
+    red[kPar][wave][lane] = acc;
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the weights stay in flight
+    __builtin_amdgcn_s_barrier();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    const int b = 4 * grp + wave;
+    const float *part = reinterpret_cast<const float *>(&red[kPar][0][lane]) + wave;
+    float y = part[0];
+#pragma unroll
+    for (int k = 1; k < 4; k++) y += part[k * 256];
+    if (b < a.B) a.out[(size_t)b * a.out_ld + g * 16 + col] = y * sc;
+  };
+  int g = blockIdx.x;
+  load(0, g);
+  for (; g < tiles; g += 2 * gridDim.x) {
+    step(g, std::integral_constant<int, 0>{});
+    if (g + (int)gridDim.x < tiles) step(g + gridDim.x, std::integral_constant<int, 1>{});
   }
 }
 
@@ -879,9 +945,29 @@ unsigned blocks_for(size_t n) { return (unsigned)((n + kThreads - 1) / kThreads)
 
 }  // namespace
 
+// K = 256 kL up to kL = kMaxRegsL.
+constexpr int kMaxRegsL = 12;
+
+template <int kL>
+hipError_t launch_gemv_regs_l(hipStream_t s, const GemvArgs &a) {
+  if constexpr (kL > kMaxRegsL) {
+    return hipErrorInvalidValue;
+  } else {
+    if (a.K != 256 * kL) return launch_gemv_regs_l<kL + 1>(s, a);
+    // as many workgroups as are resident together (3 or 2 per CU), so that a
+    // workgroup's activations are loaded once for several tiles
+    const int grid = std::min(a.N / 16, kL <= 4 ? 768 : 512);
+    gemv_regs_kernel<kL><<<grid, kThreads, 0, s>>>(a);
+    return hipGetLastError();
+  }
+}
+
 hipError_t launch_gemv(hipStream_t s, const GemvArgs &a_in, int weight_type, int pro, int epi,
                        int max_grid) {
   GemvArgs a = a_in;
+  if (weight_type == kWeightFp8 && pro == kProNone && epi == kEpiStore && !a.bias && a.scale &&
+      a.K <= 256 * kMaxRegsL && a.K % 256 == 0)
+    return launch_gemv_regs_l<1>(s, a);
   const int groups = a.N / (16 * (epi == kEpiSwiGLU ? 2 : 1));
   // split K over the 4 waves of a workgroup, one tile group per workgroup
   // (grid-striding past max_grid)
