@@ -129,36 +129,96 @@ __global__ __launch_bounds__(kT) void gelu_kernel(const float *__restrict__ x, f
 
 // ---- argmax ------------------------------------------------------------------
 
-// Key of x[i]: larger values give larger keys, NaN the largest of all (as
-// numpy's argmax, which returns the first NaN), and among equal keys the
-// smaller index wins.
-__device__ __forceinline__ unsigned long long argmax_key_nan(float v, int i) {
-  return v != v ? (0xffffffffull << 32) | (unsigned long long)(0xffffffffu - (uint32_t)i)
-                : argmax_key(v, i);
+// Order of the values: argmax_key's (its high word here), by which -0 lies
+// below +0; NaN, of either sign, above everything (as numpy's argmax, which
+// returns the first NaN). Equal values: the smaller index.
+__device__ __forceinline__ uint32_t order_key(uint32_t u) {
+  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
-// grid (rows): index[row] = the first position of the row's maximum.
-__global__ __launch_bounds__(kT) void argmax_kernel(const float *__restrict__ x, int n,
-                                                    int32_t *__restrict__ index) {
-  __shared__ unsigned long long red[4];
-  const float *xr = x + (size_t)blockIdx.x * n;
-  unsigned long long best = 0;
-  for (int i = threadIdx.x; i < n; i += kT) {
-    const unsigned long long k = argmax_key_nan(xr[i], i);
-    best = k > best ? k : best;
-  }
+// The largest of a, b, c; -0 < +0. Of no use where one of them is NaN.
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
+constexpr int kArgT = 1024;
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
+// Minimum over the workgroup of kArgT threads, in every thread.
+__device__ __forceinline__ uint32_t block_min_u32(uint32_t v, uint32_t *red) {
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    const unsigned long long o = __shfl_xor(best, off, 64);
-    best = o > best ? o : best;
-  }
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = best;
+  for (int off = 32; off >= 1; off >>= 1) v = min(v, (uint32_t)__shfl_xor((int)v, off, 64));
+  __syncthreads();  // red's earlier readers are done
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long k = red[0];
-    for (int w = 1; w < 4; w++) k = red[w] > k ? red[w] : k;
-    index[blockIdx.x] = (int32_t)(0xffffffffu - (uint32_t)(k & 0xffffffffu));
+  v = red[0];
+#pragma unroll
+  for (int w = 1; w < kArgT / 64; w++) v = min(v, red[w]);
+  return v;
+}
+
+// grid (rows): index[row] = the first position of the row's maximum. One
+// workgroup of 16 waves reads a row, 8 vectors of 4 values in flight per
+// thread, so a row streams at what one CU can load. A vector's maximum is
+// found as floats and only that compared (as its order key) with the thread's
+// best, whose vector is remembered; the position within it is looked up at the
+// end. A row that holds a NaN is scanned again for the first one. 16 rows of
+// 151936: 189 us with 4 waves per row, one value and one 64-bit key comparison
+// at a time; 8.5 us a pass here.
+__global__ __launch_bounds__(kArgT) void argmax_kernel(const float *__restrict__ x, int n,
+                                                       int32_t *__restrict__ index) {
+  constexpr int kU = 8;
+  __shared__ uint32_t red[kArgT / 64];
+  const float *xr = x + (size_t)blockIdx.x * n;
+  const int t = threadIdx.x;
+  uint32_t best = 0;  // below every value's key
+  int at = 0;         // first position of the best vector
+  bool nan = false;
+  // vectors at 0, 4, .., the last one at n - 4 (clamped starts: a vector read
+  // twice changes nothing)
+  if (n >= 4) {
+    for (int v0 = 4 * t; v0 < n; v0 += 4 * kArgT * kU) {
+      f32x4 v[kU];
+#pragma unroll
+      for (int u = 0; u < kU; u++)
+        v[u] = *reinterpret_cast<const f32x4_any *>(xr + min(v0 + 4 * kArgT * u, n - 4));
+#pragma unroll
+      for (int u = 0; u < kU; u++) {
+        nan |= __builtin_isunordered(v[u].x, v[u].y) | __builtin_isunordered(v[u].z, v[u].w);
+        const float m = max3(max3(v[u].x, v[u].y, v[u].z), v[u].w, v[u].w);
+        const uint32_t k = order_key(__builtin_bit_cast(uint32_t, m));
+        const bool better = k > best;
+        best = better ? k : best;
+        at = better ? min(v0 + 4 * kArgT * u, n - 4) : at;
+      }
+    }
+  } else if (t < n) {
+    const float m = xr[t];
+    nan = m != m;
+    best = order_key(__builtin_bit_cast(uint32_t, m));
+    at = t;
   }
+  if (__syncthreads_or(nan)) {
+    uint32_t first = 0xffffffffu;
+    for (int i = t; i < n && first == 0xffffffffu; i += kArgT)
+      if (xr[i] != xr[i]) first = (uint32_t)i;
+    first = block_min_u32(first, red);
+    if (t == 0) index[blockIdx.x] = (int32_t)first;
+    return;
+  }
+  const uint32_t top = ~block_min_u32(~best, red);
+  uint32_t first = 0xffffffffu;
+  if (best == top) {
+#pragma unroll
+    for (int e = 3; e >= 0; e--) {
+      const int i = min(at + e, n - 1);
+      if (order_key(__builtin_bit_cast(uint32_t, xr[i])) == top) first = (uint32_t)i;
+    }
+  }
+  first = block_min_u32(first, red);
+  if (t == 0) index[blockIdx.x] = (int32_t)first;
 }
 
 // ---- decode attention ----------------------------------------------------------
@@ -502,7 +562,7 @@ SH_API int sh_argmax_f32(sh_ctx *ctx, const float *x, int rows, int n, int32_t *
   if ((rc = check_range(ctx, x, (size_t)rows * n * 4, "x")) ||
       (rc = check_range(ctx, index, (size_t)rows * 4, "index")))
     return rc;
-  argmax_kernel<<<rows, kT, 0, stream_of(ctx)>>>(x, n, index);
+  argmax_kernel<<<rows, kArgT, 0, stream_of(ctx)>>>(x, n, index);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? SH_OK : hip_fail(e, "argmax");
 }
