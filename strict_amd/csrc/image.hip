@@ -4,17 +4,15 @@
 // BlurInteriorPixel / BlurEdgePixel at :85-141, in-bounds taps, sum / count),
 // plus brightness fused into the blur's row loads.
 //
-// RGBA fast path (channels == 4, width % 4 == 0, 16-byte aligned buffers): a
+// Large RGBA images in config mode (width % 4 == 0, 16-byte aligned buffers): a
 // register-streaming kernel in which each wave walks down a column strip
-// (described above the kernel). Any other shape takes a direct kernel (one
-// pixel per thread, taps read through the cache), which is exact for every
-// channel count and mode.
+// (described above the kernel). Everything else takes the byte-strip kernel,
+// which is exact for every channel count, width, alignment and mode.
 #include <hip/hip_runtime.h>
 
 #include "common.h"
 #include "swar.h"
 
-#include <cstdlib>
 
 namespace sh {
 namespace {
@@ -160,20 +158,14 @@ struct StreamArgs {
 // bias). floor(s / 25) = (s * 671089) >> 24 exactly for s < 6400: 671089 /
 // 2^24 exceeds 1/25 by < 2.2e-8, the product fits 32 bits and the quotient is
 // its top byte, which v_perm gathers.
-template <int kMode>
-__device__ __forceinline__ uint32_t finish_pixel(uint32_t vl, uint32_t vh, uint32_t count) {
-  if (kMode == SH_BLUR_CONFIG || count == 25) {
-    const uint32_t r = __umul24(vl & 0xffffu, 671089u);
-    const uint32_t b = __umul24(vl >> 16, 671089u);
-    const uint32_t g = __umul24(vh & 0xffffu, 671089u);
-    const uint32_t a = __umul24(vh >> 16, 671089u);
-    const uint32_t rg = __builtin_amdgcn_perm(g, r, 0x0c0c0703u);
-    const uint32_t ba = __builtin_amdgcn_perm(a, b, 0x07030c0cu);
-    return rg | ba;
-  }
-  const uint32_t c0 = (vl & 0xffffu) / count, c2 = (vl >> 16) / count;
-  const uint32_t c1 = (vh & 0xffffu) / count, c3 = (vh >> 16) / count;
-  return c0 | (c1 << 8) | (c2 << 16) | (c3 << 24);
+__device__ __forceinline__ uint32_t div25_pixel(uint32_t vl, uint32_t vh) {
+  const uint32_t r = __umul24(vl & 0xffffu, 671089u);
+  const uint32_t b = __umul24(vl >> 16, 671089u);
+  const uint32_t g = __umul24(vh & 0xffffu, 671089u);
+  const uint32_t a = __umul24(vh >> 16, 671089u);
+  const uint32_t rg = __builtin_amdgcn_perm(g, r, 0x0c0c0703u);
+  const uint32_t ba = __builtin_amdgcn_perm(a, b, 0x07030c0cu);
+  return rg | ba;
 }
 
 // One input row for this lane (a cached load: the band above and below read
@@ -182,16 +174,9 @@ __device__ __forceinline__ uint32_t finish_pixel(uint32_t vl, uint32_t vh, uint3
 // chunk lies outside the image load a valid chunk nobody uses (the edge fix-up
 // in hsum supplies the clamped or zero taps instead).
 
-// This lane's 4 pixels of one input row as 16-bit lanes, brightened (kFuse);
-// reference mode: rows outside the image contribute nothing.
-template <int kMode, int kFuse>
-__device__ __forceinline__ void expand_row(const u32x4 v, int y, int height, uint32_t e[8],
-                                           uint32_t d_lo, uint32_t d_hi) {
-  if (kMode == SH_BLUR_REFERENCE && (y < 0 || y >= height)) {
-#pragma unroll
-    for (int k = 0; k < 8; k++) e[k] = 0;
-    return;
-  }
+// This lane's 4 pixels of one input row as 16-bit lanes, brightened (kFuse).
+template <int kFuse>
+__device__ __forceinline__ void expand_row(const u32x4 v, uint32_t e[8], uint32_t d_lo, uint32_t d_hi) {
   const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
   for (int k = 0; k < 4; k++) {
@@ -210,7 +195,7 @@ __device__ __forceinline__ void expand_row(const u32x4 v, int y, int height, uin
 // neighbours reach their shared rows together (both at the start or both at
 // the end of the sweep; a band's bottom halo read at the end of a downward
 // sweep would be long evicted from L2 by the time the band below started).
-template <int kMode, int kFuse, int kR>
+template <int kFuse, int kR>
 __global__ __launch_bounds__(kBlurBlock) void blur_rgba_rows_kernel(const StreamArgs a) {
   constexpr int kQ = 5;  // the window's rows
   // rows requested ahead of their use (7 and 9 measured slower: their
@@ -259,13 +244,7 @@ __global__ __launch_bounds__(kBlurBlock) void blur_rgba_rows_kernel(const Stream
   // edge rule (a wave-uniform branch around eight selects per row)
   const bool edge_wave = x0 == 0 || x0 + kStripPx >= a.width;
 
-  int cxk[4];
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int x = cx + k;
-    cxk[k] = min(x + 2, a.width - 1) - max(x - 2, 0) + 1;
-  }
-  const uint32_t bias = kMode == SH_BLUR_CONFIG ? 0x000c000cu : 0u;
+  const uint32_t bias = 0x000c000cu;
   uint32_t vs[8], hs[4];
 #pragma unroll
   for (int k = 0; k < 8; k++) vs[k] = 0;
@@ -288,12 +267,7 @@ __global__ __launch_bounds__(kBlurBlock) void blur_rgba_rows_kernel(const Stream
     return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(in_rsrc, hxl * 4,
                                                                           row_offset(y), 0));
   };
-  auto expand_halo = [&](const u32x2 v, int y, uint32_t e[4]) {
-    if (kMode == SH_BLUR_REFERENCE && (y < 0 || y >= a.height)) {
-#pragma unroll
-      for (int k = 0; k < 4; k++) e[k] = 0;
-      return;
-    }
+  auto expand_halo = [&](const u32x2 v, uint32_t e[4]) {
     const uint32_t w[2] = {v.x, v.y};
 #pragma unroll
     for (int k = 0; k < 2; k++) {
@@ -317,8 +291,8 @@ __global__ __launch_bounds__(kBlurBlock) void blur_rgba_rows_kernel(const Stream
 #pragma unroll
   for (int i = 0; i < kR + 4; i++) {
     uint32_t e[8], eh[4];
-    expand_row<kMode, kFuse>(raw[i % kL], ys + dy * i, a.height, e, a.d_lo, a.d_hi);
-    expand_halo(hraw[i % kL], ys + dy * i, eh);
+    expand_row<kFuse>(raw[i % kL], e, a.d_lo, a.d_hi);
+    expand_halo(hraw[i % kL], eh);
     if (i + kL < kR + 4) {  // the slot is free: request the row kL steps ahead
       raw[i % kL] = load_row(ys + dy * (i + kL));
       hraw[i % kL] = load_halo(ys + dy * (i + kL));
@@ -356,8 +330,7 @@ __global__ __launch_bounds__(kBlurBlock) void blur_rgba_rows_kernel(const Stream
       lo[7] = from_right(lo[3], hs[2]);
       hi[6] = from_right(hi[2], hs[1]);
       hi[7] = from_right(hi[3], hs[3]);
-      if (!edge_wave) {
-      } else if (kMode == SH_BLUR_CONFIG) {
+      if (edge_wave) {
         lo[0] = left_edge ? lo[2] : lo[0];
         lo[1] = left_edge ? lo[2] : lo[1];
         hi[0] = left_edge ? hi[2] : hi[0];
@@ -366,15 +339,6 @@ __global__ __launch_bounds__(kBlurBlock) void blur_rgba_rows_kernel(const Stream
         lo[7] = right_edge ? lo[5] : lo[7];
         hi[6] = right_edge ? hi[5] : hi[6];
         hi[7] = right_edge ? hi[5] : hi[7];
-      } else {
-        lo[0] = left_edge ? 0u : lo[0];
-        lo[1] = left_edge ? 0u : lo[1];
-        hi[0] = left_edge ? 0u : hi[0];
-        hi[1] = left_edge ? 0u : hi[1];
-        lo[6] = right_edge ? 0u : lo[6];
-        lo[7] = right_edge ? 0u : lo[7];
-        hi[6] = right_edge ? 0u : hi[6];
-        hi[7] = right_edge ? 0u : hi[7];
       }
       uint32_t h[8];
 #pragma unroll
@@ -388,14 +352,11 @@ __global__ __launch_bounds__(kBlurBlock) void blur_rgba_rows_kernel(const Stream
         h[6 + part] = t + q[6] + q[7] + bias;
       }
       {
-        const uint32_t ry = kMode == SH_BLUR_CONFIG
-                                ? 5u
-                                : (uint32_t)(min(y + 2, a.height - 1) - max(y - 2, 0) + 1);
         u32x4 o;
-        o.x = finish_pixel<kMode>(h[0], h[1], ry * cxk[0]);
-        o.y = finish_pixel<kMode>(h[2], h[3], ry * cxk[1]);
-        o.z = finish_pixel<kMode>(h[4], h[5], ry * cxk[2]);
-        o.w = finish_pixel<kMode>(h[6], h[7], ry * cxk[3]);
+        o.x = div25_pixel(h[0], h[1]);
+        o.y = div25_pixel(h[2], h[3]);
+        o.z = div25_pixel(h[4], h[5]);
+        o.w = div25_pixel(h[6], h[7]);
         // rows past the image's bottom land past the resource's end too
         __builtin_amdgcn_raw_buffer_store_b128(
             o, out_rsrc, (int)(out_lane + (uint32_t)(row * a.width * 4)), 0, 2);  // 2: nt
@@ -432,43 +393,218 @@ __global__ __launch_bounds__(kBlock) void rgb_to_bgr_kernel(const uint8_t *__res
 }
 
 // ---------------------------------------------------------------------------
-// Blur, direct kernel for any channel count / width (one pixel per thread).
+// Blur, byte-strip kernel: 1 to 4 channels, any width and alignment.
+//
+// A row is a string of bytes whose taps lie kC bytes apart. One wave owns a
+// strip of kStripBytes output bytes and kR output rows; lane l holds the 8
+// bytes at p = strip start + 8 (l - 1), the first and the last lane being halo
+// only. All kR + 4 input rows are requested at the start, then added into the
+// 5-row column sums as 16-bit pairs (bytes 0 and 2, 1 and 3 of each of the two
+// words). A tap b bytes away is, for a pair, a pair of this or a neighbour
+// lane or the halves of two of them: lane moves by DPP and v_alignbit, no LDS.
+// Lanes at the image's left and right ends load, for each word, 8 bytes that
+// hold the clamped columns and pick them with v_perm; in reference mode the
+// outside bytes are then zeroed.
+// It took the place of one thread per pixel reading 25 taps of each channel
+// through the cache: 1919 x 1079 x 3 in reference mode 78.5 -> 7.0 us, 4096 x
+// 4096 x 3 20 us (5.0 TB/s). Bound by vector instructions (about 75 per 8 bytes
+// and row) and, below some 2 million pixels, by one round of load latency.
 // ---------------------------------------------------------------------------
 
-__global__ __launch_bounds__(kBlock) void blur_direct_kernel(const uint8_t *__restrict__ in,
-                                                             uint8_t *__restrict__ out, int width,
-                                                             int height, int channels, int mode,
-                                                             int fuse, int delta,
-                                                             int all_channels) {
-  const long long pix = (long long)blockIdx.x * kBlock + threadIdx.x;
-  if (pix >= (long long)width * height) return;
-  const int x = (int)(pix % width), y = (int)(pix / width);
-  const size_t stride = (size_t)width * channels;
-  for (int ch = 0; ch < channels; ch++) {
-    const bool adjust = fuse && (all_channels || ch < 3);
-    int sum = 0, count = 0;
-    for (int ky = -2; ky <= 2; ky++) {
-      int ny = y + ky;
-      if (mode == SH_BLUR_CONFIG) {
-        ny = min(max(ny, 0), height - 1);
-      } else if (ny < 0 || ny >= height) {
-        continue;
+constexpr int kBytesBlock = 256;
+constexpr int kStripBytes = 62 * 8;
+
+struct BytesArgs {
+  const uint8_t *in;
+  uint8_t *out;
+  size_t row_bytes;
+  int height, strips, total_waves, xcd_blocks;
+  uint32_t mag, mask;  // brightness: |delta| in every byte, bytes to adjust
+  int bright;          // 0: none, 1: add, 2: subtract
+};
+
+// Bytes b and b + 2 from this lane's first (lo: bytes 0, 2, hi: bytes 1, 3 of
+// words -2 .. 3 in [0 .. 5]).
+template <int kB>
+__device__ __forceinline__ uint32_t pair_at(const uint32_t (&lo)[6], const uint32_t (&hi)[6]) {
+  constexpr int i = (kB + 8) / 4, r = (kB + 8) % 4, j = r < 2 ? i : i + 1;
+  static_assert(kB >= -8 && j < 6, "taps reach two words");
+  if (r == 0) return lo[i];
+  if (r == 1) return hi[i];
+  return r == 2 ? __builtin_amdgcn_alignbit(lo[j], lo[i], 16) : __builtin_amdgcn_alignbit(hi[j], hi[i], 16);
+}
+
+// The five taps of bytes kB and kB + 2.
+template <int kC, int kB>
+__device__ __forceinline__ uint32_t taps5(const uint32_t (&lo)[6], const uint32_t (&hi)[6]) {
+  return pair_at<kB - 2 * kC>(lo, hi) + pair_at<kB - kC>(lo, hi) + pair_at<kB>(lo, hi) +
+         pair_at<kB + kC>(lo, hi) + pair_at<kB + 2 * kC>(lo, hi);
+}
+
+template <int kC, int kMode, int kR>
+__global__ __launch_bounds__(kBytesBlock) void blur_bytes_kernel(const BytesArgs a) {
+  typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(1)));
+  typedef uint32_t u32_any __attribute__((aligned(1)));
+  typedef uint16_t u16_any __attribute__((aligned(1)));
+  const int blk = (blockIdx.x & 7) * a.xcd_blocks + (blockIdx.x >> 3);
+  const int lane = threadIdx.x & 63;
+  const int wi = blk * (kBytesBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (wi >= a.total_waves) return;
+  const int strip = wi % a.strips, band = wi / a.strips;
+  const int y0 = band * kR;
+  const size_t s0 = (size_t)strip * kStripBytes;
+  // positions relative to the strip: this lane's first byte, the row's end
+  const int p = 8 * (lane - 1);
+  const int end = (int)min(a.row_bytes - s0, (size_t)(2 * kStripBytes));
+  const bool first = s0 == 0, edge_x = first || end < kStripBytes + 8;  // wave-uniform
+  auto row = [&](int y) {
+    return a.in + (size_t)min(max(y, 0), a.height - 1) * a.row_bytes + s0;
+  };
+
+  u32x2 raw[kR + 4];
+  u32x2 inside = {0, 0};  // reference mode, edge_x: bytes inside the image
+  if (!edge_x) {
+#pragma unroll
+    for (int i = 0; i < kR + 4; i++) raw[i] = *reinterpret_cast<const u32x2_any *>(row(y0 - 2 + i) + p);
+  } else {
+    int at[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const int b = p + k;  // >= -8
+      at[k] = b;
+      if (first && b < 0) at[k] = (b + 8 * kC) % kC;                // the first pixel's
+      if (b >= end) at[k] = end - kC + (b - end) % kC;               // the last pixel's
+      if ((b >= 0 || !first) && b < end) inside[k / 4] |= 0xffu << (8 * (k & 3));
+    }
+    if (a.row_bytes >= 8) {
+      // a word's bytes lie within 8 bytes from its own clamped position
+      int base[2];
+      uint32_t sel[2];
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        base[j] = min(first ? max(p + 4 * j, 0) : p + 4 * j, end - 8);
+        sel[j] = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) sel[j] |= (uint32_t)(at[4 * j + k] - base[j]) << (8 * k);
       }
-      for (int kx = -2; kx <= 2; kx++) {
-        int nx = x + kx;
-        if (mode == SH_BLUR_CONFIG) {
-          nx = min(max(nx, 0), width - 1);
-        } else if (nx < 0 || nx >= width) {
-          continue;
-        }
-        int v = in[(size_t)ny * stride + (size_t)nx * channels + ch];
-        if (adjust) v = min(255, max(0, v + delta));
-        sum += v;
-        count++;
+      u32x2 wide[kR + 4][2];
+#pragma unroll
+      for (int i = 0; i < kR + 4; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+          wide[i][j] = *reinterpret_cast<const u32x2_any *>(row(y0 - 2 + i) + base[j]);
+#pragma unroll
+      for (int i = 0; i < kR + 4; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+          raw[i][j] = __builtin_amdgcn_perm(wide[i][j].y, wide[i][j].x, sel[j]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < kR + 4; i++) {
+        const uint8_t *q = row(y0 - 2 + i);
+        raw[i] = u32x2{0, 0};
+#pragma unroll
+        for (int k = 0; k < 8; k++) raw[i][k / 4] |= (uint32_t)q[at[k]] << (8 * (k & 3));
       }
     }
-    const int r = mode == SH_BLUR_CONFIG ? (sum + 12) / 25 : sum / count;
-    out[(size_t)y * stride + (size_t)x * channels + ch] = (uint8_t)r;
+  }
+
+  // (brightness and the zeroing in passes of their own, so that the row loop
+  // below is straight-line code)
+  if (a.bright) {
+#pragma unroll
+    for (int i = 0; i < kR + 4; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) raw[i][j] = brighten_u8x4(raw[i][j], a.mag, a.bright == 2, a.mask);
+  }
+  const bool edge_y = y0 < 2 || y0 + kR + 2 > a.height;  // wave-uniform
+  uint32_t recip[8];
+  if (kMode == SH_BLUR_REFERENCE) {
+    if (edge_x) {
+#pragma unroll
+      for (int i = 0; i < kR + 4; i++) raw[i] &= inside;
+    }
+    if (edge_y) {
+#pragma unroll
+      for (int i = 0; i < kR + 4; i++)
+        if (y0 - 2 + i < 0 || y0 - 2 + i >= a.height) raw[i] = u32x2{0, 0};
+    }
+  }
+
+  const bool writer = lane >= 1 && lane < 63 && p < end;
+  const bool whole = p + 8 <= end;
+  uint32_t v[4] = {0, 0, 0, 0}, ring[5][4];  // column sums: lo, hi of word 0, of word 1
+#pragma unroll
+  for (int i = 0; i < kR + 4; i++) {
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const uint32_t e[2] = {__builtin_amdgcn_perm(0u, raw[i][j], 0x0c020c00u),
+                             __builtin_amdgcn_perm(0u, raw[i][j], 0x0c030c01u)};
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        v[2 * j + q] += e[q];
+        if (i >= 5) v[2 * j + q] -= ring[i % 5][2 * j + q];
+        ring[i % 5][2 * j + q] = e[q];
+      }
+    }
+    if (i < 4) continue;
+    const int y = y0 + i - 4;  // the window's centre row
+    uint32_t lo[6], hi[6];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      lo[2 + j] = v[2 * j];
+      hi[2 + j] = v[2 * j + 1];
+      lo[j] = from_left(v[2 * j], 0);
+      hi[j] = from_left(v[2 * j + 1], 0);
+      lo[4 + j] = from_right(v[2 * j], 0);
+      hi[4 + j] = from_right(v[2 * j + 1], 0);
+    }
+    const uint32_t bias = kMode == SH_BLUR_CONFIG ? 0x000c000cu : 0u;
+    const uint32_t sum[4] = {taps5<kC, 0>(lo, hi) + bias, taps5<kC, 1>(lo, hi) + bias,
+                             taps5<kC, 4>(lo, hi) + bias, taps5<kC, 5>(lo, hi) + bias};
+    u32x2 o;
+    if (kMode == SH_BLUR_CONFIG || !(edge_x || edge_y)) {
+      o = u32x2{div25_pixel(sum[0], sum[1]), div25_pixel(sum[2], sum[3])};
+    } else {
+      // floor(s / n) = (s m) >> 24 for s <= 255 n, 2 <= n <= 25 in-bounds taps (a
+      // 1 x 1 image runs in config mode) and 2^24 / n <= m < 2^24 / n + 4: the
+      // product stays below 2^32 and exceeds s 2^24 / n by less than 2^24 / n.
+      // v_rcp_f32's 1 ulp leaves 2^24 / n within 1, the conversion within 2
+      const int ry = max(min(y + 2, a.height - 1) - max(y - 2, 0) + 1, 1);
+      if (i == 4 || edge_y) {
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+          const int b = p + k;
+          const int left = first ? min(max(b, 0) / kC, 2) : 2, right = min(max(end - 1 - b, 0) / kC, 2);
+          const int rx = left + 1 + right;
+          recip[k] = (uint32_t)(16777216.0f * __builtin_amdgcn_rcpf((float)(rx * ry))) + 2;
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        const uint32_t q0 = __umul24(sum[2 * j] & 0xffffu, recip[4 * j]);
+        const uint32_t q2 = __umul24(sum[2 * j] >> 16, recip[4 * j + 2]);
+        const uint32_t q1 = __umul24(sum[2 * j + 1] & 0xffffu, recip[4 * j + 1]);
+        const uint32_t q3 = __umul24(sum[2 * j + 1] >> 16, recip[4 * j + 3]);
+        o[j] = __builtin_amdgcn_perm(q1, q0, 0x0c0c0703u) | __builtin_amdgcn_perm(q3, q2, 0x07030c0cu);
+      }
+    }
+    uint8_t *q = a.out + (size_t)y * a.row_bytes + s0 + p;
+    if (writer && whole && y < a.height) *reinterpret_cast<u32x2_any *>(q) = o;
+    if (edge_x && writer && !whole && y < a.height) {
+      // the row's last bytes: 4, 2 and 1 of them
+      const int n = end - p;
+      uint32_t w = o.x;
+      if (n & 4) {
+        *reinterpret_cast<u32_any *>(q) = w;
+        w = o.y;
+      }
+      if (n & 2) {
+        *reinterpret_cast<u16_any *>(q + (n & 4)) = (uint16_t)w;
+        w >>= 16;
+      }
+      if (n & 1) q[n - 1] = (uint8_t)w;
+    }
   }
 }
 
@@ -489,20 +625,9 @@ Brightness make_brightness(bool enabled, int channels, int delta, int all_channe
 // two rounds).
 constexpr int kBlurRows = 16;
 
-template <int kMode, int kR>
-void launch_rows_fuse(hipStream_t s, const StreamArgs &a, int fuse) {
-  const int blocks = a.xcd_blocks * 8;
-  if (fuse == 1)
-    blur_rgba_rows_kernel<kMode, 1, kR><<<blocks, kBlurBlock, 0, s>>>(a);
-  else if (fuse == 2)
-    blur_rgba_rows_kernel<kMode, 2, kR><<<blocks, kBlurBlock, 0, s>>>(a);
-  else
-    blur_rgba_rows_kernel<kMode, 0, kR><<<blocks, kBlurBlock, 0, s>>>(a);
-}
-
 template <int kRowsPerWave>
 void launch_blur_stream(hipStream_t s, const uint32_t *in, uint32_t *out, int width, int height,
-                        int mode, bool fuse, int delta, int all_channels) {
+                        bool fuse, int delta, int all_channels) {
   StreamArgs a;
   a.in = in;
   a.out = out;
@@ -523,10 +648,43 @@ void launch_blur_stream(hipStream_t s, const uint32_t *in, uint32_t *out, int wi
     a.d_lo = d | (d << 16);                                 // R and B
     a.d_hi = d | (all_channels ? d << 16 : 0u);             // G, and A only if asked
   }
-  if (mode == SH_BLUR_CONFIG)
-    launch_rows_fuse<SH_BLUR_CONFIG, kRowsPerWave>(s, a, f);
+  if (f == 1)
+    blur_rgba_rows_kernel<1, kRowsPerWave><<<blocks, kBlurBlock, 0, s>>>(a);
+  else if (f == 2)
+    blur_rgba_rows_kernel<2, kRowsPerWave><<<blocks, kBlurBlock, 0, s>>>(a);
   else
-    launch_rows_fuse<SH_BLUR_REFERENCE, kRowsPerWave>(s, a, f);
+    blur_rgba_rows_kernel<0, kRowsPerWave><<<blocks, kBlurBlock, 0, s>>>(a);
+}
+
+template <int kC, int kMode, int kR>
+void launch_blur_bytes(hipStream_t s, const BytesArgs &a) {
+  // padded to 8 workgroups so that every XCD gets an equal range of bands
+  const int blocks = ((a.total_waves + kBytesBlock / 64 - 1) / (kBytesBlock / 64) + 7) / 8 * 8;
+  BytesArgs b = a;
+  b.xcd_blocks = blocks / 8;
+  blur_bytes_kernel<kC, kMode, kR><<<blocks, kBytesBlock, 0, s>>>(b);
+}
+
+template <int kC>
+void launch_blur_channels(hipStream_t s, BytesArgs a, int mode) {
+  a.strips = (int)((a.row_bytes + kStripBytes - 1) / kStripBytes);
+  // 4 rows per wave keep the chip full at ordinary sizes (1919 x 1079 x 3: 7.0 us
+  // against 8.6 with 8 rows); where there are waves enough, 8 rows re-read
+  // fewer (4095 x 4095 x 4: 25.3 against 28.8)
+  const long long waves8 = (long long)a.strips * ((a.height + 7) / 8);
+  const int rows = waves8 >= 12000 ? 8 : 4;
+  a.total_waves = a.strips * ((a.height + rows - 1) / rows);
+  if (mode == SH_BLUR_CONFIG) {
+    if (rows == 8)
+      launch_blur_bytes<kC, SH_BLUR_CONFIG, 8>(s, a);
+    else
+      launch_blur_bytes<kC, SH_BLUR_CONFIG, 4>(s, a);
+  } else {
+    if (rows == 8)
+      launch_blur_bytes<kC, SH_BLUR_REFERENCE, 8>(s, a);
+    else
+      launch_blur_bytes<kC, SH_BLUR_REFERENCE, 4>(s, a);
+  }
 }
 
 }  // namespace
@@ -549,14 +707,32 @@ hipError_t launch_brightness_u8(hipStream_t s, const uint8_t *in, uint8_t *out, 
 
 hipError_t launch_blur5_u8(hipStream_t s, const uint8_t *in, uint8_t *out, int width, int height,
                            int channels, int mode, bool fuse, int delta, int all_channels) {
-  if (channels == 4 && width % 4 == 0 && aligned16(in) && aligned16(out)) {
+  // The streaming kernel for large aligned RGBA images in config mode: 3840 x
+  // 2160 11.4 us against the byte strips' 15.5, 3000 x 2000 9.5 against 10.3; with
+  // fewer pixels its 16 rows per wave leave most of the chip idle: 2400 x 1600
+  // 10.7 against 9.9, 1920 x 1080 9.2 against 5.8, 512 x 512 17.7 against 4.6
+  if (mode == SH_BLUR_CONFIG && channels == 4 && width % 4 == 0 && aligned16(in) && aligned16(out) &&
+      (long long)width * height >= 5000000) {
     const uint32_t *in32 = reinterpret_cast<const uint32_t *>(in);
     uint32_t *out32 = reinterpret_cast<uint32_t *>(out);
-    launch_blur_stream<kBlurRows>(s, in32, out32, width, height, mode, fuse, delta, all_channels);
-  } else {
-    const long long pixels = (long long)width * height;
-    blur_direct_kernel<<<(unsigned)((pixels + kBlock - 1) / kBlock), kBlock, 0, s>>>(
-        in, out, width, height, channels, mode, fuse ? 1 : 0, delta, all_channels);
+    launch_blur_stream<kBlurRows>(s, in32, out32, width, height, fuse, delta, all_channels);
+    return hipGetLastError();
+  }
+  BytesArgs a;
+  a.in = in;
+  a.out = out;
+  a.height = height;
+  a.row_bytes = (size_t)width * channels;
+  const Brightness br = make_brightness(fuse, channels, delta, all_channels);
+  a.mag = br.mag;
+  a.mask = br.mask;
+  a.bright = !fuse || delta == 0 ? 0 : br.negative ? 2 : 1;
+  if (width == 1 && height == 1) mode = SH_BLUR_CONFIG;  // both give the pixel itself
+  switch (channels) {
+    case 1: launch_blur_channels<1>(s, a, mode); break;
+    case 2: launch_blur_channels<2>(s, a, mode); break;
+    case 3: launch_blur_channels<3>(s, a, mode); break;
+    default: launch_blur_channels<4>(s, a, mode); break;
   }
   return hipGetLastError();
 }
