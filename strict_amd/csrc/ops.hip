@@ -11,17 +11,18 @@
 // points of the oracle (oracle/llm.py).
 //
 // Decode attention is split-K flash decoding: grid (split, KV head, row),
-// each workgroup streams its split's positions in 64-position tiles of K and
-// V through LDS with a running softmax (max, sum, unnormalised V sum) per
-// query head, and writes those three as a partial; a merge kernel per
-// (row, head) combines the partials. The partials live in a work buffer:
-// the context's (sh_attn_decode_f16) or a fixed device array
+// each workgroup takes its split's positions with a running softmax (max,
+// sum, unnormalised V sum) per query head, and writes those three as a
+// partial; a merge kernel per (row, head) combines the partials (with one
+// split the first kernel writes the output). The partials live in a work
+// buffer: the context's (sh_attn_decode_f16) or a fixed device array
 // (sh_attn_decode_f16_noalloc).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 
 #include "common.h"
 #include "llm_device.h"
@@ -223,8 +224,9 @@ __global__ __launch_bounds__(kArgT) void argmax_kernel(const float *__restrict__
 
 // ---- decode attention ----------------------------------------------------------
 
-constexpr int kTile = 64;      // positions per K / V tile
 constexpr int kMaxGroup = 16;  // query heads per KV head
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+#define SH_OPS_LDS __attribute__((address_space(3)))
 
 struct AttnOpArgs {
   const float *q;            // [B][heads][d]
@@ -236,145 +238,358 @@ struct AttnOpArgs {
   float scale;
 };
 
-// grid (splits, kv_heads, B): positions [s * chunk, min((s + 1) * chunk, L))
-// of row b for the G = heads / kv_heads query heads of KV head kvh.
+// Positions whose K and V a workgroup requests at once (64 KiB): 8 loads of 16
+// bytes of each per thread.
 template <int kD>
-__global__ __launch_bounds__(kT) void attn_op_partials_kernel(const AttnOpArgs a) {
-  constexpr int kRow = kD + 8;                        // padded LDS row of K (fp16)
-  constexpr int kAcc = kMaxGroup * kD / kT;           // (head, dim) pairs per thread
-  constexpr int kHeadsPerWave = kMaxGroup / 4;
-  __shared__ float qs[kMaxGroup][kD];
-  __shared__ __attribute__((aligned(16))) _Float16 ks[kTile][kRow];
-  __shared__ __attribute__((aligned(16))) _Float16 vs[kTile][kD];
-  __shared__ float ps[kMaxGroup][kTile];
-  __shared__ float corr[kMaxGroup];
+constexpr int kAttnTile = 8 * 256 * 8 / kD;
+
+// exp(x) for x <= 0 to about 1 ulp: x log2(e) in two parts, the small one as a
+// factor.
+__device__ __forceinline__ float exp_neg(float x) {
+  constexpr float kL = 1.44269502f, kLo = 1.92596299e-8f;  // log2(e) = kL + kLo
+  const float hi = x * kL;
+  const float lo = fmaf(x, kLo, fmaf(x, kL, -hi));
+  const float e = __builtin_amdgcn_exp2f(hi);
+  return x > -150.0f ? fmaf(e * 0.693147181f, lo, e) : x != x ? x : 0.0f;
+}
+
+// grid (splits, kv_heads, B): positions [s * chunk, min((s + 1) * chunk, L)) of
+// row b for the G = heads / kv_heads query heads of KV head kvh, in tiles of
+// kAttnTile positions. The kernel is bound by the K and V bytes, so all of a
+// tile's loads are issued before any is used, and no wave waits for another in
+// the loop: each takes a quarter of the tile's positions and keeps a running
+// softmax (maximum, sum and V sum per head) of its own; the four are combined
+// at the end. The arithmetic is MFMA's, whatever G is (the unused columns cost
+// nothing that is missed):
+//  - scores as K x q: K fragments straight from memory (a lane: 8 dims of
+//    position lane % 16), heads in the columns; a lane then holds 4 consecutive
+//    positions of each 16-position block for head lane % 16;
+//  - V sums as V^T x P, the k slots numbered as P has them (slot (g, e):
+//    position 4 g + e of the first block for e < 4, of the second for e >= 4);
+//    V goes through LDS rows as it is and comes back by transposing reads.
+// q and P stay fp32 to 2^-22: q as two fp16 after an exact power-of-two scaling
+// of each head to below 1, P times 2^14 as two fp16. (Error against 64 bits
+// 2.6e-7; the fp32 kernel before it, 64-position tiles staged in LDS with one
+// serial V sum per thread, 4.1e-7.)
+// Measured, both kernels of a call, before and after: 4 rows up to 4,096
+// positions, 16 / 8 heads of 128: 29.7 -> 13.5 us (50 MB, 3.7 TB/s); 16 rows 68.3
+// -> 38.5 (4.7 TB/s); 16 rows of 8,192, 16 / 1 heads 73.7 -> 25.2; 1 row of 384,
+// 12 / 12 heads of 64 9.0 -> 8.2. fp32 FMAs from registers in its place were as
+// fast at one query head per KV head and slower from two on (16 / 1 heads: 65.8).
+template <int kD>
+__global__ __launch_bounds__(kT, 3) void attn_op_partials_kernel(const AttnOpArgs a) {
+  constexpr int kKK = kD / 32, kDT = kD / 16;
+  constexpr int kBlocks = kAttnTile<kD> / 4 / 16;  // 16-position blocks per wave and tile
+  constexpr int kVLoads = kBlocks * 16 * kD / 8 / 64;
+  constexpr int kRow = kD * 2, kChunks = kD / 8;   // a V row in LDS: bytes, 16-byte chunks
+  constexpr float kPScale = 16384.0f;
+  union Lds {
+    uint8_t v[4][kBlocks * 16 * kRow];
+    float acc[4][kMaxGroup][kD];
+    float q[kMaxGroup][kD];
+  };
+  __shared__ __attribute__((aligned(16))) Lds lds;
+  __shared__ __attribute__((aligned(16))) _Float16 qh[2][kMaxGroup][kD + 8];
+  __shared__ float qscale[kMaxGroup], stat[4][kMaxGroup][2];
 
   const int s = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int r16 = lane & 15, grp = lane >> 4;
   const int G = a.heads / a.kv_heads;
   const int L = min(a.lengths[b], a.max_pos);
   const int p0 = s * a.chunk;
-  if (p0 >= L) return;  // uniform: nothing of this row in the split
-  const int p1 = min(p0 + a.chunk, L);
   const int h0 = kvh * G;
-
-  for (int i = t; i < G * kD; i += kT)
-    qs[i / kD][i % kD] = a.q[((size_t)b * a.heads + h0 + i / kD) * kD + i % kD] * a.scale;
-
-  float m_run[kHeadsPerWave], l_run[kHeadsPerWave];
-#pragma unroll
-  for (int j = 0; j < kHeadsPerWave; j++) {
-    m_run[j] = -INFINITY;
-    l_run[j] = 0.0f;
+  if (p0 >= L) {  // uniform: nothing of this row in the split
+    if (a.splits == 1)
+      for (int i = t; i < G * kD; i += kT) a.out[((size_t)b * a.heads + h0) * kD + i] = 0.0f;
+    return;
   }
-  float acc[kAcc];
-#pragma unroll
-  for (int j = 0; j < kAcc; j++) acc[j] = 0.0f;
+  const int p1 = min(p0 + a.chunk, L);
 
   const size_t row0 = ((size_t)b * a.kv_heads + kvh) * (size_t)a.max_pos;
-  const uint16_t *kb = a.k + row0 * kD;
-  const uint16_t *vb = a.v + row0 * kD;
-  for (int pt = p0; pt < p1; pt += kTile) {
-    const int n = min(kTile, p1 - pt);
-    __syncthreads();  // the previous tile's LDS reads are done (and qs is written)
-    // K and V rows of the tile in 16-byte vectors; rows past n re-read the
-    // tile's last position (in bounds, never weighted)
-    for (int vi = t; vi < kTile * kD / 8; vi += kT) {
-      const int r = vi / (kD / 8), c8 = (vi % (kD / 8)) * 8;
-      const size_t p = (size_t)min(pt + r, p1 - 1);
-      *reinterpret_cast<u32x4 *>(&ks[r][c8]) = *reinterpret_cast<const u32x4 *>(kb + p * kD + c8);
-      *reinterpret_cast<u32x4 *>(&vs[r][c8]) = *reinterpret_cast<const u32x4 *>(vb + p * kD + c8);
+  const uint16_t *kb = a.k + row0 * kD + grp * 8;
+  const uint16_t *vb = a.v + row0 * kD + (lane % kChunks) * 8;
+  f16x8 kf[kBlocks][kKK];
+  u32x4 vr[kVLoads];
+  // positions past the split re-read its last one (never weighted)
+  auto load_k = [&](int pt) __attribute__((always_inline)) {
+    const int pw = pt + wave * (16 * kBlocks);
+#pragma unroll
+    for (int tt = 0; tt < kBlocks; tt++)
+#pragma unroll
+      for (int kk = 0; kk < kKK; kk++)
+        kf[tt][kk] = *reinterpret_cast<const f16x8 *>(
+            kb + (size_t)min(pw + 16 * tt + r16, p1 - 1) * kD + 32 * kk);
+  };
+  auto load_v = [&](int pt) __attribute__((always_inline)) {
+    const int pw = pt + wave * (16 * kBlocks);
+#pragma unroll
+    for (int u = 0; u < kVLoads; u++)
+      vr[u] = *reinterpret_cast<const u32x4 *>(
+          vb + (size_t)min(pw + (u * 64 + lane) / kChunks, p1 - 1) * kD);
+  };
+  // q is requested ahead of K and V, so that waiting for it does not wait for them
+  constexpr int kQ = kMaxGroup * kD / kT;
+  float q[kQ];
+#pragma unroll
+  for (int u = 0; u < kQ; u++)
+    q[u] = a.q[((size_t)b * a.heads + h0) * kD + min(t + kT * u, G * kD - 1)];
+  __builtin_amdgcn_sched_barrier(0);
+  load_k(p0);
+  load_v(p0);
+  __builtin_amdgcn_sched_barrier(0);
+  auto lds_barrier = [] {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): K and V stay in flight
+    __builtin_amdgcn_s_barrier();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  };
+#pragma unroll
+  for (int u = 0; u < kQ; u++)
+    if (t + kT * u < G * kD) (&lds.q[0][0])[t + kT * u] = q[u] * a.scale;
+  lds_barrier();
+  for (int g = wave; g < G; g += 4) {
+    float x[kD / 64], mx = 0.0f;
+#pragma unroll
+    for (int e = 0; e < kD / 64; e++) {
+      x[e] = lds.q[g][lane + 64 * e];
+      mx = fmaxf(mx, fabsf(x[e]));
     }
-    __syncthreads();
-    // scores: wave w holds heads w, w + 4, ..; lane = position in the tile
+    mx = wave_max_rows(mx);
+    // 2^ex > mx >= 2^(ex - 1) (0 for zero, infinity and NaN)
+    const int ex = min(max(__builtin_amdgcn_frexp_expf(mx), -120), 120);
+    if (lane == 0) qscale[g] = ldexpf(1.0f, ex);
 #pragma unroll
-    for (int j = 0; j < kHeadsPerWave; j++) {
-      const int g = wave + 4 * j;
-      if (g >= G) break;  // wave-uniform
-      float dot = 0.0f;
-#pragma unroll
-      for (int c = 0; c < kD; c += 8) {
-        const f16x8 kk = *reinterpret_cast<const f16x8 *>(&ks[lane][c]);
-#pragma unroll
-        for (int e = 0; e < 8; e++) dot += qs[g][c + e] * (float)kk[e];
-      }
-      const bool valid = lane < n;
-      const float sc = valid ? dot : -INFINITY;
-      const float m_new = fmaxf(m_run[j], wave_max(sc));
-      const float pr = valid ? expf(sc - m_new) : 0.0f;
-      const float c_old = expf(m_run[j] - m_new);  // 0 on the first tile
-      l_run[j] = l_run[j] * c_old + wave_sum(pr);
-      m_run[j] = m_new;
-      ps[g][lane] = pr;
-      if (lane == 0) corr[g] = c_old;
-    }
-    __syncthreads();
-    // V sums: thread t owns (head, dim) pairs t, t + 256, ..
-#pragma unroll
-    for (int j = 0; j < kAcc; j++) {
-      const int idx = t + kT * j, g = idx / kD, dd = idx % kD;
-      if (g < G) {
-        float sum = 0.0f;
-#pragma unroll 8
-        for (int p = 0; p < kTile; p++) sum += ps[g][p] * (float)vs[p][dd];
-        acc[j] = acc[j] * corr[g] + sum;
-      }
+    for (int e = 0; e < kD / 64; e++) {
+      const float y = ldexpf(x[e], -ex);
+      const _Float16 hi = (_Float16)y;
+      qh[0][g][lane + 64 * e] = hi;
+      qh[1][g][lane + 64 * e] = (_Float16)(y - (float)hi);
     }
   }
-  // partials of this split
+  lds_barrier();
+  const float qs = qscale[min(r16, G - 1)];  // (columns past G repeat the last head, unused)
+
+  float m_run = -INFINITY, l_run = 0.0f;
+  f32x4 acc[kDT];
+#pragma unroll
+  for (int dt = 0; dt < kDT; dt++) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  uint8_t *vl = lds.v[wave];
+  // chunk c of row r lies at c ^ 2 f(r): a transposing read's 32 lanes (8 rows,
+  // 2 chunks each) then hit 64 banks
+  auto swz = [](int r) { return kD == 128 ? 2 * (r & 7) : 2 * ((r >> 1) & 3); };
+  // (more_c: another tile follows; its K is requested as soon as the scores have
+  // used this one's, its V as soon as this one's is in LDS)
+  auto tile = [&](int pt, auto more_c) __attribute__((always_inline)) {
+    constexpr bool kMore = decltype(more_c)::value;
+    f32x4 sc[kBlocks];
+#pragma unroll
+    for (int tt = 0; tt < kBlocks; tt++) sc[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < kKK; kk++)
+#pragma unroll
+      for (int part = 0; part < 2; part++) {
+        const f16x8 qf = *reinterpret_cast<const f16x8 *>(&qh[part][min(r16, G - 1)][32 * kk + 8 * grp]);
+#pragma unroll
+        for (int tt = 0; tt < kBlocks; tt++)
+          sc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[tt][kk], qf, sc[tt], 0, 0, 0);
+      }
+    if constexpr (kMore) {
+      __builtin_amdgcn_sched_barrier(0);
+      load_k(pt + kAttnTile<kD>);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // V to this wave's LDS rows (LDS works in order: after the last tile's reads)
+#pragma unroll
+    for (int u = 0; u < kVLoads; u++) {
+      const int r = (u * 64 + lane) / kChunks, c = lane % kChunks;
+      *reinterpret_cast<u32x4 *>(vl + r * kRow + ((c ^ swz(r)) * 16)) = vr[u];
+    }
+    if constexpr (kMore) {
+      __builtin_amdgcn_sched_barrier(0);
+      load_v(pt + kAttnTile<kD>);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    float mx = -INFINITY;
+    const int pw = pt + wave * (16 * kBlocks) + 4 * grp;
+#pragma unroll
+    for (int tt = 0; tt < kBlocks; tt++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        sc[tt][e] = pw + 16 * tt + e < p1 ? sc[tt][e] * qs : -INFINITY;
+        mx = fmaxf(mx, sc[tt][e]);
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float m = fmaxf(m_run, mx);
+    const float corr = m_run == m ? 1.0f : exp_neg(m_run - m);
+    m_run = m;
+    float ls = 0.0f;
+    f16x8 p[kBlocks / 2][2];
+#pragma unroll
+    for (int tt = 0; tt < kBlocks; tt++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float w = pw + 16 * tt + e < p1 ? exp_neg(sc[tt][e] - m) * kPScale : 0.0f;
+        const _Float16 hi = (_Float16)w;
+        p[tt / 2][0][(tt & 1) * 4 + e] = hi;
+        p[tt / 2][1][(tt & 1) * 4 + e] = (_Float16)(w - (float)hi);
+        ls += w;
+      }
+    l_run = l_run * corr + ls;  // this lane's positions; the groups are summed at the end
+#pragma unroll
+    for (int dt = 0; dt < kDT; dt++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) acc[dt][e] *= corr;
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // this wave's V rows are in LDS
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    const int ti = (lane >> 2) & 3, tq = lane & 3;
+#pragma unroll
+    for (int sl = 0; sl < kBlocks / 2; sl++)
+#pragma unroll
+      for (int dt = 0; dt < kDT; dt++) {
+        s16x4 half[2];
+#pragma unroll
+        for (int q2 = 0; q2 < 2; q2++) {
+          const int r = 32 * sl + 16 * q2 + 4 * grp + ti, c = 2 * dt + (tq >> 1);
+          half[q2] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (SH_OPS_LDS s16x4 *)((SH_OPS_LDS uint8_t *)vl + r * kRow + ((c ^ swz(r)) * 16) + (tq & 1) * 8));
+        }
+        const f16x8 vf = __builtin_bit_cast(
+            f16x8, __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+        for (int part = 0; part < 2; part++)
+          acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, p[sl][part], acc[dt], 0, 0, 0);
+      }
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  };
+  int pt = p0;
+  for (; pt + kAttnTile<kD> < p1; pt += kAttnTile<kD>) tile(pt, std::true_type{});
+  tile(pt, std::false_type{});
+
+  l_run += __shfl_xor(l_run, 16, 64);
+  l_run += __shfl_xor(l_run, 32, 64);
+  if (grp == 0) {
+    stat[wave][r16][0] = m_run;
+    stat[wave][r16][1] = l_run;
+  }
+  lds_barrier();  // every wave's V reads are done: lds.v becomes lds.acc
+  if (r16 < G) {
+#pragma unroll
+    for (int dt = 0; dt < kDT; dt++)
+      *reinterpret_cast<f32x4 *>(&lds.acc[wave][r16][16 * dt + 4 * grp]) = acc[dt];
+  }
+  lds_barrier();
+  // the split's partial: the four waves' sums against their common maximum
   const size_t pstride = (size_t)kD + 2;
+  for (int i = t; i < G * kD; i += kT) {
+    const int g = i / kD, dd = i % kD;
+    float m = stat[0][g][0];
 #pragma unroll
-  for (int j = 0; j < kAcc; j++) {
-    const int idx = t + kT * j, g = idx / kD, dd = idx % kD;
-    if (g < G)
-      a.part[(((size_t)b * a.heads + h0 + g) * a.splits + s) * pstride + dd] = acc[j];
-  }
-  if (lane == 0) {
+    for (int w = 1; w < 4; w++) m = fmaxf(m, stat[w][g][0]);
+    float sum = 0.0f, l = 0.0f;
 #pragma unroll
-    for (int j = 0; j < kHeadsPerWave; j++) {
-      const int g = wave + 4 * j;
-      if (g < G) {
-        float *pp = a.part + (((size_t)b * a.heads + h0 + g) * a.splits + s) * pstride + kD;
-        pp[0] = m_run[j];
-        pp[1] = l_run[j];
-      }
+    for (int w = 0; w < 4; w++) {
+      const float f = stat[w][g][0] == m ? 1.0f : exp_neg(stat[w][g][0] - m);
+      sum = fmaf(f, lds.acc[w][g][dd], sum);
+      l = fmaf(f, stat[w][g][1], l);
+    }
+    if (a.splits == 1) {  // the whole row: no merge follows
+      a.out[((size_t)b * a.heads + h0) * kD + i] = sum / l;
+      continue;
+    }
+    float *pp = a.part + (((size_t)b * a.heads + h0 + g) * a.splits + s) * pstride;
+    pp[dd] = sum;
+    if (dd == 0) {
+      pp[kD] = m;
+      pp[kD + 1] = l;
     }
   }
 }
 
-// grid (heads, B), kD threads:
+// grid (heads, B), 4 kD threads:
 //   out = sum_j exp(m_j - M) acc_j / sum_j exp(m_j - M) l_j,  M = max_j m_j
-// over the row's active splits j (rows of length <= 0: zeros).
+// over the row's active splits j (rows of length <= 0: zeros). Thread (part,
+// dim) takes splits part, part + 4, .. against their own maximum, 8 requested
+// at once; the four parts are combined at the end.
+constexpr int kMergeParts = 4;
 template <int kD>
-__global__ __launch_bounds__(kD) void attn_op_merge_kernel(const AttnOpArgs a) {
-  const int h = blockIdx.x, b = blockIdx.y, i = threadIdx.x;
+__global__ __launch_bounds__(kD * kMergeParts) void attn_op_merge_kernel(const AttnOpArgs a) {
+  constexpr int kStep = 8;
+  __shared__ float red[kMergeParts][kD], lred[kMergeParts], mred[kMergeParts];
+  const int h = blockIdx.x, b = blockIdx.y, t = threadIdx.x, i = t % kD, part = t / kD;
   const int L = min(a.lengths[b], a.max_pos);
   float *o = a.out + ((size_t)b * a.heads + h) * kD;
   if (L <= 0) {
-    o[i] = 0.0f;
+    if (part == 0) o[i] = 0.0f;
     return;
   }
   const int active = (L + a.chunk - 1) / a.chunk;
   const size_t pstride = (size_t)kD + 2;
   const float *pp = a.part + ((size_t)b * a.heads + h) * a.splits * pstride;
-  float M = -INFINITY;
-  for (int j = 0; j < active; j++) M = fmaxf(M, pp[(size_t)j * pstride + kD]);
-  float num = 0.0f, den = 0.0f;
-  for (int j = 0; j < active; j++) {
-    const float w = expf(pp[(size_t)j * pstride + kD] - M);
-    num += w * pp[(size_t)j * pstride + i];
-    den += w * pp[(size_t)j * pstride + kD + 1];
+  float M = -INFINITY, num = 0.0f, den = 0.0f;
+  for (int j0 = part; j0 < active; j0 += kMergeParts * kStep) {
+    float x[kStep], m[kStep], l[kStep], top = M;
+#pragma unroll
+    for (int u = 0; u < kStep; u++) {
+      const float *p = pp + (size_t)min(j0 + kMergeParts * u, active - 1) * pstride;
+      x[u] = p[i];
+      m[u] = p[kD];
+      l[u] = p[kD + 1];
+    }
+#pragma unroll
+    for (int u = 0; u < kStep; u++)
+      if (j0 + kMergeParts * u < active) top = fmaxf(top, m[u]);
+    const float c = M == top ? 1.0f : exp_neg(M - top);
+    M = top;
+    num *= c;
+    den *= c;
+#pragma unroll
+    for (int u = 0; u < kStep; u++) {
+      const float w = j0 + kMergeParts * u < active ? (m[u] == M ? 1.0f : exp_neg(m[u] - M)) : 0.0f;
+      num = fmaf(w, x[u], num);
+      den = fmaf(w, l[u], den);
+    }
+  }
+  red[part][i] = num;
+  if (i == 0) {
+    lred[part] = den;
+    mred[part] = M;
+  }
+  __syncthreads();
+  if (part != 0) return;
+  const float top = fmaxf(fmaxf(mred[0], mred[1]), fmaxf(mred[2], mred[3]));
+  num = den = 0.0f;
+#pragma unroll
+  for (int w = 0; w < kMergeParts; w++) {
+    const float f = mred[w] == top ? 1.0f : exp_neg(mred[w] - top);
+    num = fmaf(f, red[w][i], num);
+    den = fmaf(f, lred[w], den);
   }
   o[i] = num / den;
 }
 
-// Split layout of a call: about two workgroups per CU of 256, splits of
-// whole 64-position tiles.
-void attn_split(int batch, int kv_heads, int max_pos, int *splits, int *chunk) {
+// Split layout of a call. The lengths are on the device, so the splits cover
+// max_pos; one of no active position ends at once. Splits of one tile, up to
+// about 2,048 workgroups (all resident together), of more tiles beyond that;
+// where the partials of that layout would exceed the allocation-free entry's
+// array, the coarser one of about two workgroups per CU.
+void attn_split(int batch, int heads, int kv_heads, int head_dim, int max_pos, int *splits, int *chunk) {
   const long long rows = (long long)batch * kv_heads;
+  const int tile = head_dim == 64 ? kAttnTile<64> : kAttnTile<128>;
+  const long long tiles = (max_pos + tile - 1) / tile;
+  const long long per = std::max(1LL, (tiles * rows + 2047) / 2048);
+  const long long fine = (tiles + per - 1) / per;
+  if (fine <= 1024 && (long long)batch * heads * fine * (head_dim + 2) * 4 <=
+                          (long long)SH_ATTN_NOALLOC_MAX_BYTES) {
+    *chunk = (int)(per * tile);
+    *splits = (int)fine;
+    return;
+  }
   const int want = (int)std::max(1LL, std::min(1024LL, (512 + rows - 1) / rows));
   int c = (max_pos + want - 1) / want;
-  c = (c + kTile - 1) / kTile * kTile;
+  c = (c + 63) / 64 * 64;
   *chunk = c;
   *splits = (max_pos + c - 1) / c;
 }
@@ -409,16 +624,16 @@ int check_attn(sh_ctx *ctx, const float *q, const uint16_t *k, const uint16_t *v
   return SH_OK;
 }
 
-hipError_t launch_attn(hipStream_t st, AttnOpArgs a, int batch, int head_dim) {
+template <int kD>
+hipError_t launch_attn_d(hipStream_t st, const AttnOpArgs &a, int batch) {
   const dim3 grid_p(a.splits, a.kv_heads, batch), grid_m(a.heads, batch);
-  if (head_dim == 64) {
-    attn_op_partials_kernel<64><<<grid_p, kT, 0, st>>>(a);
-    attn_op_merge_kernel<64><<<grid_m, 64, 0, st>>>(a);
-  } else {
-    attn_op_partials_kernel<128><<<grid_p, kT, 0, st>>>(a);
-    attn_op_merge_kernel<128><<<grid_m, 128, 0, st>>>(a);
-  }
+  attn_op_partials_kernel<kD><<<grid_p, kT, 0, st>>>(a);
+  if (a.splits > 1) attn_op_merge_kernel<kD><<<grid_m, kD * kMergeParts, 0, st>>>(a);
   return hipGetLastError();
+}
+
+hipError_t launch_attn(hipStream_t st, const AttnOpArgs &a, int batch, int head_dim) {
+  return head_dim == 64 ? launch_attn_d<64>(st, a, batch) : launch_attn_d<128>(st, a, batch);
 }
 
 int run_attn(sh_ctx *ctx, const float *q, const uint16_t *k, const uint16_t *v,
@@ -575,7 +790,7 @@ SH_API int sh_attn_decode_f16(sh_ctx *ctx, const float *q, const uint16_t *k, co
   if ((rc = check_attn(ctx, q, k, v, lengths, out, batch, heads, kv_heads, head_dim, max_positions)))
     return rc;
   int splits = 0, chunk = 0;
-  attn_split(batch, kv_heads, max_positions, &splits, &chunk);
+  attn_split(batch, heads, kv_heads, head_dim, max_positions, &splits, &chunk);
   void *part = nullptr;
   if ((rc = context_scratch(ctx, attn_part_bytes(batch, heads, head_dim, splits), &part))) return rc;
   return run_attn(ctx, q, k, v, lengths, out, batch, heads, kv_heads, head_dim, max_positions, scale,
@@ -591,7 +806,7 @@ SH_API int sh_attn_decode_f16_noalloc(sh_ctx *ctx, const float *q, const uint16_
   if ((rc = check_attn(ctx, q, k, v, lengths, out, batch, heads, kv_heads, head_dim, max_positions)))
     return rc;
   int splits = 0, chunk = 0;
-  attn_split(batch, kv_heads, max_positions, &splits, &chunk);
+  attn_split(batch, heads, kv_heads, head_dim, max_positions, &splits, &chunk);
   const size_t need = attn_part_bytes(batch, heads, head_dim, splits);
   if (need > kNoAllocScratchBytes)
     return fail(SH_ERR_INVALID_ARGUMENT,
