@@ -265,6 +265,22 @@ hipError_t launch_gemv(hipStream_t s, const GemvArgs &a, int weight_type, int pr
                        int max_grid);
 hipError_t launch_attention(hipStream_t s, const AttnArgs &a, int head_dim, int group, bool qwen,
                             int batch);
+// The tokens a step embeds, for rows b < B.
+struct StepTokens {
+  int B = 0;
+  int t[kMaxBatch] = {};
+};
+hipError_t launch_set_tokens(hipStream_t s, unsigned long long *keys, const StepTokens &tokens);
+// Empty sequences: both key sets, the lengths and the attention counters
+// cleared; the layers kernels' step number and error words (those that exist).
+struct ResetArgs {
+  unsigned long long *keys = nullptr;
+  int *lens = nullptr, *counters = nullptr;
+  int n_lens = 0, n_counters = 0;
+  unsigned *epoch = nullptr, epoch_value = 0;
+  unsigned *err[2] = {nullptr, nullptr};
+};
+hipError_t launch_reset(hipStream_t s, const ResetArgs &a);
 hipError_t launch_embed(hipStream_t s, const EmbedArgs &a, int batch);
 // fp16 out16[b] = norm(x[b]) (pro = kProRms or kProLayer), K <= 4096.
 hipError_t launch_norm_rows(hipStream_t s, const GemvArgs &a, int pro);

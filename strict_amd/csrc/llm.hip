@@ -1003,15 +1003,19 @@ SH_API int sh_llm_reset(sh_llm *m, int batch) {
   if (batch < 1 || batch > m->cfg.max_batch)
     return fail(SH_ERR_INVALID_ARGUMENT, "batch %d outside 1..%d", batch, m->cfg.max_batch);
   hipStream_t s = stream_of(m->ctx);
-  SH_HIP_TRY(hipMemsetAsync(m->lens, 0, (size_t)m->cfg.max_batch * 4, s));
-  SH_HIP_TRY(hipMemsetAsync(m->keys, 0, (size_t)2 * kKeySet * 8, s));
-  if (m->epoch) {
-    // the device's step number to the mirror's: a layers kernel whose wait
-    // timed out may have ended before storing it (tags only ever grow)
-    SH_HIP_TRY(hipMemcpyAsync(m->epoch, &m->epoch_host, 4, hipMemcpyHostToDevice, s));
-    SH_HIP_TRY(hipStreamSynchronize(s));
-  }
-  SH_HIP_TRY(hipMemsetAsync(m->counters, 0, (size_t)m->cfg.max_batch * m->cfg.kv_heads * 4, s));
+  ResetArgs r;
+  r.keys = m->keys;
+  r.lens = m->lens;
+  r.n_lens = m->cfg.max_batch;
+  r.counters = m->counters;
+  r.n_counters = m->cfg.max_batch * m->cfg.kv_heads;
+  // the device's step number to the mirror's: a layers kernel whose wait
+  // timed out may have ended before storing it (tags only ever grow)
+  r.epoch = m->epoch;
+  r.epoch_value = m->epoch_host;
+  r.err[0] = m->layers_kernel ? m->la.err : nullptr;
+  r.err[1] = m->gpt2_kernel ? m->ga.err : nullptr;
+  SH_HIP_TRY(launch_reset(s, r));
   m->batch = batch;
   m->splits = attention_splits(batch, m->cfg.kv_heads, m->cfg.max_positions);
   m->chunk = ((m->cfg.max_positions + m->splits - 1) / m->splits + 15) / 16 * 16;
@@ -1036,12 +1040,10 @@ SH_API int sh_llm_reset(sh_llm *m, int batch) {
     const char *xe = getenv("STRICT_HIP_LLM_XCD");
     a.xcd = !(xe && xe[0] == '0') && !m->xcd_off && decode_layers_xcd_ok(a, m->layers_grid) ? 1 : 0;
     m->layers_lds = decode_layers_lds(batch, c.hidden, c.heads, c.intermediate, &a.lds_misc);
-    SH_HIP_TRY(hipMemsetAsync(a.err, 0, 4, s));
   }
   if (m->gpt2_kernel) {
     const char *xe = getenv("STRICT_HIP_LLM_XCD");
     m->ga.xcd = !(xe && xe[0] == '0') && !m->xcd_off && gpt2_layers_xcd_ok(m->ga, m->gpt2_grid) ? 1 : 0;
-    SH_HIP_TRY(hipMemsetAsync(m->ga.err, 0, 4, s));
   }
   return SH_OK;
 }
@@ -1055,15 +1057,14 @@ SH_API int sh_llm_step(sh_llm *m, const int32_t *tokens, int want_logits) {
     return fail(SH_ERR_INVALID_ARGUMENT, "KV cache full (%d positions)", m->cfg.max_positions);
   hipStream_t s = stream_of(m->ctx);
   if (tokens) {
-    // the token in slot 0, every other slot cleared (a previous head's keys)
-    unsigned long long keys[kKeySlots * kKeyStride] = {};
+    StepTokens st;
+    st.B = m->batch;
     for (int b = 0; b < m->batch; b++) {
       if (tokens[b] < 0 || tokens[b] >= m->cfg.vocab)
         return fail(SH_ERR_INVALID_ARGUMENT, "token %d of row %d outside the vocabulary", tokens[b], b);
-      keys[b] = (unsigned long long)(0xffffffffu - (uint32_t)tokens[b]);
+      st.t[b] = tokens[b];
     }
-    SH_HIP_TRY(hipMemcpyAsync(key_set(m), keys, sizeof(keys), hipMemcpyHostToDevice, s));
-    SH_HIP_TRY(hipStreamSynchronize(s));  // `keys` is a stack array
+    SH_HIP_TRY(launch_set_tokens(s, key_set(m), st));
   }
   const int g = want_logits ? 1 : 0;
   if (!m->use_graphs || m->layers_kernel || (m->gpt2_kernel && m->batch == 1)) {

@@ -889,6 +889,35 @@ __global__ __launch_bounds__(kThreads) void embed_kernel(const EmbedArgs a) {
   }
 }
 
+// ---- step state written by the host ------------------------------------------
+// The values travel as kernel arguments: a copy from host memory would make the
+// host wait for the stream, and the GPU for the host, before every step.
+
+// One workgroup: key set `keys` holds tokens[b] in slot 0 of row b < B, every
+// other key cleared (a previous head's).
+__global__ __launch_bounds__(kThreads) void set_tokens_kernel(unsigned long long *keys, StepTokens tokens) {
+  for (int i = threadIdx.x; i < kKeySet; i += kThreads) {
+    unsigned long long k = 0;
+#pragma unroll
+    for (int b = 0; b < kMaxBatch; b++)
+      if (i == b && b < tokens.B) k = (unsigned long long)(0xffffffffu - (uint32_t)tokens.t[b]);
+    keys[i] = k;
+  }
+}
+
+// One workgroup: empty sequences (see ResetArgs).
+__global__ __launch_bounds__(kThreads) void reset_kernel(const ResetArgs a) {
+  const int t = threadIdx.x;
+  for (int i = t; i < 2 * kKeySet; i += kThreads) a.keys[i] = 0;
+  for (int i = t; i < a.n_lens; i += kThreads) a.lens[i] = 0;
+  for (int i = t; i < a.n_counters; i += kThreads) a.counters[i] = 0;
+  if (t == 0) {
+    if (a.epoch) *a.epoch = a.epoch_value;
+    if (a.err[0]) *a.err[0] = 0;
+    if (a.err[1]) *a.err[1] = 0;
+  }
+}
+
 size_t gemv_lds_bytes(const GemvArgs &a, int pro) {
   size_t lds = (size_t)a.B * (a.K + 8) * 2 + 4 * 2 * 64 * 4 * sizeof(float);
   if (pro != kProNone) lds += (size_t)a.B * a.K * 4 + 2 * (size_t)a.K * 4;
@@ -1034,6 +1063,16 @@ hipError_t launch_norm_rows(hipStream_t s, const GemvArgs &a, int pro) {
     norm_rows_kernel<kProLayer><<<a.B, kThreads, 0, s>>>(a);
   else
     norm_rows_kernel<kProRms><<<a.B, kThreads, 0, s>>>(a);
+  return hipGetLastError();
+}
+
+hipError_t launch_set_tokens(hipStream_t s, unsigned long long *keys, const StepTokens &tokens) {
+  set_tokens_kernel<<<1, kThreads, 0, s>>>(keys, tokens);
+  return hipGetLastError();
+}
+
+hipError_t launch_reset(hipStream_t s, const ResetArgs &a) {
+  reset_kernel<<<1, kThreads, 0, s>>>(a);
   return hipGetLastError();
 }
 
