@@ -78,6 +78,16 @@ __device__ __forceinline__ float wave_max_rows(float v) {
 
 __device__ __forceinline__ float silu(float x) { return x / (1.0f + expf(-x)); }
 
+// exp(x) for x <= 0 to about 1 ulp: x log2(e) in two parts, the small one as a
+// factor.
+__device__ __forceinline__ float exp_neg(float x) {
+  constexpr float kL = 1.44269502f, kLo = 1.92596299e-8f;  // log2(e) = kL + kLo
+  const float hi = x * kL;
+  const float lo = fmaf(x, kLo, fmaf(x, kL, -hi));
+  const float e = __builtin_amdgcn_exp2f(hi);
+  return x > -150.0f ? fmaf(e * 0.693147181f, lo, e) : x != x ? x : 0.0f;
+}
+
 // Order-preserving key of an fp32 logit with its column: larger logits give
 // larger keys; among equal logits the smaller column wins (as argmax does).
 __device__ __forceinline__ unsigned long long argmax_key(float v, int n) {

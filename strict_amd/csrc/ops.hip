@@ -421,16 +421,6 @@ struct AttnOpArgs {
 template <int kD>
 constexpr int kAttnTile = 8 * 256 * 8 / kD;
 
-// exp(x) for x <= 0 to about 1 ulp: x log2(e) in two parts, the small one as a
-// factor.
-__device__ __forceinline__ float exp_neg(float x) {
-  constexpr float kL = 1.44269502f, kLo = 1.92596299e-8f;  // log2(e) = kL + kLo
-  const float hi = x * kL;
-  const float lo = fmaf(x, kLo, fmaf(x, kL, -hi));
-  const float e = __builtin_amdgcn_exp2f(hi);
-  return x > -150.0f ? fmaf(e * 0.693147181f, lo, e) : x != x ? x : 0.0f;
-}
-
 // grid (splits, kv_heads, B): positions [s * chunk, min((s + 1) * chunk, L)) of
 // row b for the G = heads / kv_heads query heads of KV head kvh, in tiles of
 // kAttnTile positions. The kernel is bound by the K and V bytes, so all of a

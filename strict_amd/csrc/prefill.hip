@@ -14,6 +14,8 @@
 // is in the batch.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "common.h"
 #include "llm.h"
 #include "llm_device.h"
@@ -82,6 +84,16 @@ __global__ void prefill_finish_kernel(int *lens, int B, int n) {
 
 // ---- linears -------------------------------------------------------------------
 
+// Groups of 4 waves that share a tile's K stages (every kGroups-th each); fixed
+// per epilogue, so that a sum's order is. Two where the outputs are few (the
+// residual linears, N = hidden): their stages are a serial chain on a chip that
+// is not full. O and down, 1,023 tokens of 1024 x 2048 and 1024 x 3072: 15.0 and
+// 21.4 us with one group, 11.2 and 15.2 with two; 128 tokens of 768 x 3072 23.7
+// and 18.6; 4,090 tokens 35 and 48, 29 and 39; 8,000 tokens of 768 x 768 17.6
+// and 19.0. The wide linears lose by it once the chip is full: QKV at 4,090
+// tokens 56 and 71 us, gate / up at 1,023 23.9 and 27.5.
+constexpr int groups_of(int epi) { return epi == kEpiResidual ? 2 : 1; }
+
 // C[m][n] = sum_k A[m][k] W[n][k], then the epilogue. A: fp16 rows; W: tiled
 // weights (N a multiple of 64, K of 128). A workgroup owns 32 kMI tokens x
 // 32 kMI outputs as 2 x 2 waves of kMI x kMI MFMA tiles. K advances in 64-wide
@@ -92,21 +104,23 @@ __global__ void prefill_finish_kernel(int *lens, int B, int n) {
 // issued as W x A, which leaves a lane with 4 consecutive outputs of one
 // token (16-byte fp32, 8-byte fp16 stores).
 template <int kW, int kEpi, int kMI>
-__global__ __launch_bounds__(kT, kMI == 4 ? 2 : 4) void prefill_gemm_kernel(const PrefillGemmArgs g, int tiles_m,
-                                                          int ntiles, int per_xcd) {
-  constexpr int kBM = 32 * kMI;
+__global__ __launch_bounds__(kT * groups_of(kEpi), kMI == 4 ? 2 : 4) void prefill_gemm_kernel(
+    const PrefillGemmArgs g, int tiles_m, int ntiles, int per_xcd) {
+  constexpr int kBM = 32 * kMI, kGroups = groups_of(kEpi);
   constexpr int kChunks = kBM * 8 / kT;            // 16-byte chunks per thread and stage
   constexpr int kWL = kW == kWeightFp8 ? 1 : 2;    // 16-byte weight loads per tile and stage
-  __shared__ __attribute__((aligned(16))) uint8_t lds[2][kBM * 128];
+  __shared__ __attribute__((aligned(16))) uint8_t lds_all[kGroups][2][kBM * 128];
   // each XCD takes a run of tiles, tokens fastest: its L2 then reads few
   // weight rows, once
   const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if (tile >= ntiles) return;
   const int tm = tile % tiles_m, tn = tile / tiles_m;
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int group = __builtin_amdgcn_readfirstlane(threadIdx.x / kT);
+  const int t = threadIdx.x % kT, lane = t & 63, wave = t >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int m0 = tm * kBM, nt0 = tn * 2 * kMI + wn * kMI;  // first 16-row weight tile of the wave
   const int K = g.K, nk = K / 64;
+  uint8_t (*lds)[kBM * 128] = lds_all[group];
 
   const uint16_t *arow[kChunks];
   int aoff[kChunks];
@@ -166,39 +180,62 @@ __global__ __launch_bounds__(kT, kMI == 4 ? 2 : 4) void prefill_gemm_kernel(cons
     }
   };
 
-  load_a(0, 0);
-  load_w(0, 0);
-  load_a(1, 1);  // nk >= 2
-  load_w(1, 1);
+  // this group's stages: group, group + kGroups, ..; nk is a multiple of
+  // kGroups. Iteration it uses set / buffer it % 2; the next stage's rows go to
+  // the other buffer, which every wave has finished reading (the barrier that
+  // ended the previous iteration). (The order is kept: a store moved up ahead of
+  // the loads would wait for the stage requested last, not the one before it.)
+  const int nit = nk / kGroups;
+  auto stage = [&](int it) { return min(it, nit - 1) * kGroups + group; };  // past the end: unused
+  auto step = [&](int it, auto par_c) __attribute__((always_inline)) {
+    constexpr int kPar = decltype(par_c)::value;
+    load_a(kPar, stage(it + 2));
+    __builtin_amdgcn_sched_barrier(0);
+    compute(kPar, kPar);
+    load_w(kPar, stage(it + 2));
+    __builtin_amdgcn_sched_barrier(0);
+    store_a(kPar ^ 1, kPar ^ 1);
+    lds_barrier();
+  };
+  load_a(0, stage(0));
+  load_w(0, stage(0));
+  load_a(1, stage(1));
+  load_w(1, stage(1));
   store_a(0, 0);
   lds_barrier();
-  // stage kt (even part: set / buffer 0, odd part: 1); the next stage's rows
-  // go to the other buffer, which every wave has finished reading (the
-  // barrier that ended the previous stage)
-  for (int kt = 0; kt < nk; kt += 2) {
-    const int k2 = min(kt + 2, nk - 1), k3 = min(kt + 3, nk - 1);  // past the end: re-read, unused
-    // (the order is kept: a store moved up ahead of the loads would wait for
-    // the stage requested last, not the one before it)
-    load_a(0, k2);
-    __builtin_amdgcn_sched_barrier(0);
-    compute(0, 0);
-    load_w(0, k2);
-    __builtin_amdgcn_sched_barrier(0);
-    store_a(1, 1);
+  int it = 0;
+  for (; it + 1 < nit; it += 2) {
+    step(it, std::integral_constant<int, 0>{});
+    step(it + 1, std::integral_constant<int, 1>{});
+  }
+  if (it < nit) step(it, std::integral_constant<int, 0>{});
+
+  // the groups' sums: group q finishes the q-th part of the wave's token tiles
+  constexpr int kOwn = kMI / kGroups;
+  if constexpr (kGroups == 2) {
+    f32x4 *red = reinterpret_cast<f32x4 *>(&lds_all[0][0][0]);  // [from group][i][j][thread]
+#pragma unroll
+    for (int i = 0; i < kOwn; i++)
+#pragma unroll
+      for (int j = 0; j < kMI; j++) {
+        const f32x4 give = group == 0 ? acc[kOwn + i][j] : acc[i][j];
+        red[((group * kOwn + i) * kMI + j) * kT + t] = give;
+      }
     lds_barrier();
-    load_a(1, k3);
-    __builtin_amdgcn_sched_barrier(0);
-    compute(1, 1);
-    load_w(1, k3);
-    __builtin_amdgcn_sched_barrier(0);
-    store_a(0, 0);
-    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < kOwn; i++)
+#pragma unroll
+      for (int j = 0; j < kMI; j++) {
+        const f32x4 x = red[(((group ^ 1) * kOwn + i) * kMI + j) * kT + t];
+        const f32x4 own = group == 0 ? acc[i][j] : acc[kOwn + i][j];
+        acc[i][j] = f32x4{own[0] + x[0], own[1] + x[1], own[2] + x[2], own[3] + x[3]};
+      }
   }
 
   const int nl = 4 * (lane >> 4);  // this lane's 4 outputs within a 16-row tile
 #pragma unroll
-  for (int i = 0; i < kMI; i++) {
-    const int m = m0 + frow + 16 * i;
+  for (int i = 0; i < kOwn; i++) {
+    const int m = m0 + frow + 16 * (group * kOwn + i);
     if (m >= g.M) continue;
 #pragma unroll
     for (int j = 0; j < kMI; j++) {
@@ -322,11 +359,18 @@ __global__ __launch_bounds__(kT) void prefill_qkv_kernel(const PrefillArgs a, in
 
 // ---- causal attention ---------------------------------------------------------------
 
-constexpr int kKeys = 64;  // positions per K / V tile
+constexpr int kAttnT = 512;
 
-// grid (ceil(T / (64 kQT)), heads, B): 64 kQT tokens of one head against the
-// cache, 16 kQT per wave; tiles of 64 positions from position 0, so that a
-// token's running softmax passes over the same tiles whatever chunk it is in.
+// Key parts of an attention tile, fixed per head size: 32 positions each.
+constexpr int attn_parts(int d) { return d == 128 ? 4 : 2; }
+// Tokens per workgroup: the 8 waves are parts x groups of 16 tokens.
+constexpr int attn_tokens(int d) { return 128 / attn_parts(d); }
+
+// grid (heads, ceil(T / attn_tokens), B): a block of tokens of one head against
+// the cache. Tiles of 32 kKP positions start at position 0 and a part is a
+// fixed 32 of each, so a token's kKP running softmaxes pass over the same
+// positions whatever chunk of the prompt it is in; they are merged in one order
+// at the end.
 //  - scores as K x q: a lane holds one token (lane % 16) and 4 consecutive
 //    positions of each 16-position tile, so the softmax's row maximum needs
 //    two lane moves and the exponentials are the P operand in place;
@@ -337,37 +381,60 @@ constexpr int kKeys = 64;  // positions per K / V tile
 // kSplit: q and P as two fp16 each (22 bits), for the models whose decode
 // steps keep both in fp32; otherwise one fp16 each, the softmax sum taken
 // over the rounded P, as the decode-layers kernel does.
-template <int kD, bool kVT, bool kSplit, int kQT>
-__global__ __launch_bounds__(kT) void prefill_attn_kernel(const PrefillArgs a) {
-  constexpr int kKRow = kD + 8, kVRow = kKeys + 4;  // padded LDS rows (fp16)
+//
+// What bounds it is a tile's way from the L2 through LDS to the MFMAs, step
+// after step behind barriers: of 22.3 us at 1,023 tokens of 16 heads of 128 the
+// loads and LDS stores alone take 14.5, all but the loads 18.5. So the keys of
+// a tile are split over waves (4 waves of 16 tokens on a 64-position tile:
+// 37.5 us, 400 at 4,090 tokens; now 23 and 222) and two workgroups share a CU,
+// one's loads beside the other's MFMAs. 64 tokens per workgroup with half the
+// K and V traffic but one workgroup per CU: 26 us, 266 at 4,090 tokens.
+// Fragments straight from the cache, no LDS and no barrier: 32 us.
+template <int kD, bool kVT, bool kSplit>
+__global__ __launch_bounds__(kAttnT, kSplit && kD == 128 ? 2 : 4) void prefill_attn_kernel(
+    const PrefillArgs a) {
+  constexpr int kKP = attn_parts(kD), kKeys = 32 * kKP, kGroupsT = 8 / kKP;
+  // padded LDS rows (fp16): 16 rows on 16 different bank groups
+  constexpr int kKRow = kD + 8, kVRow = kKeys + 8;
   constexpr int kKK = kD / 32, kDT = kD / 16;
-  constexpr int kLoads = kKeys * kD / 8 / kT;  // 16-byte loads per thread, tile and operand
+  constexpr int kLoads = kKeys * kD / 8 / kAttnT;  // 16-byte loads per thread, tile and operand
   constexpr int kParts = kSplit ? 2 : 1;
-  __shared__ __attribute__((aligned(16))) _Float16 ks[kKeys * kKRow];
-  __shared__ __attribute__((aligned(16))) _Float16 vs[kD * kVRow];
+  __shared__ __attribute__((aligned(16))) union {
+    struct {
+      _Float16 k[kKeys * kKRow], v[kD * kVRow];
+    } tile;
+    f32x4 acc[kKP][kGroupsT][kDT][64];
+  } lds;
+  __shared__ float stat[kKP][kGroupsT][2][64];  // maximum, sum
+  _Float16 *ks = lds.tile.k, *vs = lds.tile.v;
 
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((t >> 6) % kGroupsT);  // token group
+  const int kh = __builtin_amdgcn_readfirstlane((t >> 6) / kGroupsT);    // key part
   const int r = lane & 15, grp = lane >> 4;
-  const int h = blockIdx.y, b = blockIdx.z, kvh = h / (a.heads / a.kv_heads);
-  const int q0 = (gridDim.x - 1 - blockIdx.x) * 64 * kQT;  // the longest first
+  // workgroups x, x + kv_heads, .. share a KV head: with 8 of those an XCD's L2
+  // holds the one it works on
+  const int kvh = blockIdx.x % a.kv_heads, b = blockIdx.z;
+  const int h = kvh * (a.heads / a.kv_heads) + blockIdx.x / a.kv_heads;
+  // the longest half of the blocks first, longest first; then the others,
+  // shortest first: a CU's second workgroup evens out its first
+  const int blocks = gridDim.y, by = blockIdx.y, half = (blocks + 1) / 2;
+  const int q0 = attn_tokens(kD) * (by < half ? blocks - 1 - by : by - half);
   const int base = max(a.lens[b], 0) + a.i0;
-  const int kend = min(base + min(q0 + 64 * kQT, a.T), a.max_pos);  // positions any token sees
+  const int kend = min(base + min(q0 + attn_tokens(kD), a.T), a.max_pos);  // positions any token sees
 
-  int qpos[kQT];
-  size_t qrow[kQT];
-  f16x8 qf[kQT][kParts][kKK];
+  // this lane's token, and the first and the last position of the wave's tokens
+  const int w0 = q0 + 16 * wave, i = min(w0 + r, a.T - 1);
+  const int qpos = min(base + i, a.max_pos - 1);
+  const int qlo = min(base + min(w0, a.T - 1), a.max_pos - 1);
+  const int qhi = min(base + min(w0 + 15, a.T - 1), a.max_pos - 1);
+  const size_t qrow = (((size_t)b * a.T + i) * a.heads + h) * kD;
+  f16x8 qf[kParts][kKK];
 #pragma unroll
-  for (int u = 0; u < kQT; u++) {
-    const int i = min(q0 + (wave * kQT + u) * 16 + r, a.T - 1);
-    qpos[u] = min(base + i, a.max_pos - 1);
-    qrow[u] = (((size_t)b * a.T + i) * a.heads + h) * kD;
-#pragma unroll
-    for (int kk = 0; kk < kKK; kk++) {
-      qf[u][0][kk] = *reinterpret_cast<const f16x8 *>(a.q + qrow[u] + 32 * kk + 8 * grp);
-      if (kSplit)
-        qf[u][kParts - 1][kk] =
-            *reinterpret_cast<const f16x8 *>(a.q_lo + qrow[u] + 32 * kk + 8 * grp);
-    }
+  for (int kk = 0; kk < kKK; kk++) {
+    qf[0][kk] = *reinterpret_cast<const f16x8 *>(a.q + qrow + 32 * kk + 8 * grp);
+    if (kSplit)
+      qf[kParts - 1][kk] = *reinterpret_cast<const f16x8 *>(a.q_lo + qrow + 32 * kk + 8 * grp);
   }
 
   const size_t cache = (size_t)b * a.kv_heads + kvh;
@@ -376,141 +443,160 @@ __global__ __launch_bounds__(kT) void prefill_attn_kernel(const PrefillArgs a) {
   u32x4 kr[kLoads], vr[kLoads];
   // tile pt of K and V into registers, clamped to cached positions
   auto load = [&](int pt) {
+    const uint16_t *kt = kb + (size_t)pt * kD, *vt = vb + (kVT ? (size_t)pt : (size_t)pt * kD);
+    const int last = kend - 1 - pt;
 #pragma unroll
     for (int u = 0; u < kLoads; u++) {
-      const int c = t + kT * u;
-      const int p = min(pt + c / (kD / 8), kend - 1);
-      kr[u] = *reinterpret_cast<const u32x4 *>(kb + (size_t)p * kD + (c % (kD / 8)) * 8);
-      if (kVT) {  // 8 positions of one dim
-        const int dd = c >> 3, p8 = min(pt + (c & 7) * 8, (kend - 1) & ~7);
-        vr[u] = *reinterpret_cast<const u32x4 *>(vb + (size_t)dd * a.vt_stride + p8);
-      } else {  // 8 dims of one position
-        vr[u] = *reinterpret_cast<const u32x4 *>(vb + (size_t)p * kD + (c % (kD / 8)) * 8);
-      }
+      const int c = t + kAttnT * u;
+      kr[u] = *reinterpret_cast<const u32x4 *>(kt + min(c / (kD / 8), last) * kD + c % (kD / 8) * 8);
+      if (kVT)  // 8 positions of one dim
+        vr[u] = *reinterpret_cast<const u32x4 *>(
+            vt + (size_t)(c / (kKeys / 8)) * a.vt_stride + min(c % (kKeys / 8) * 8, last & ~7));
+      else  // 8 dims of one position, positions along the lanes for the transposing store
+        vr[u] = *reinterpret_cast<const u32x4 *>(vt + min(c % kKeys, last) * kD + c / kKeys * 8);
     }
   };
   auto store = [&](int pt) {
 #pragma unroll
     for (int u = 0; u < kLoads; u++) {
-      const int c = t + kT * u;
+      const int c = t + kAttnT * u;
       const int row = c / (kD / 8), c8 = (c % (kD / 8)) * 8;
       *reinterpret_cast<u32x4 *>(&ks[row * kKRow + c8]) = kr[u];
       const f16x8 v = __builtin_bit_cast(f16x8, vr[u]);
       if (kVT) {
         // positions past the cached ones may hold anything: zeros instead
         // (their P is 0, but 0 x NaN is not)
-        const int dd = c >> 3, pl = (c & 7) * 8;
-        f16x4 w[2];
+        const int dd = c / (kKeys / 8), pl = c % (kKeys / 8) * 8;
+        f16x8 w = v;
+        if (pt + kKeys > kend) {
 #pragma unroll
-        for (int e = 0; e < 8; e++) w[e >> 2][e & 3] = pt + pl + e < kend ? v[e] : (_Float16)0.0f;
-        *reinterpret_cast<f16x4 *>(&vs[dd * kVRow + pl]) = w[0];
-        *reinterpret_cast<f16x4 *>(&vs[dd * kVRow + pl + 4]) = w[1];
+          for (int e = 0; e < 8; e++) w[e] = pt + pl + e < kend ? v[e] : (_Float16)0.0f;
+        }
+        *reinterpret_cast<f16x8 *>(&vs[dd * kVRow + pl]) = w;
       } else {
+        const int pv = c % kKeys, d8 = c / kKeys * 8;
 #pragma unroll
-        for (int e = 0; e < 8; e++) vs[(c8 + e) * kVRow + row] = v[e];
+        for (int e = 0; e < 8; e++) vs[(d8 + e) * kVRow + pv] = v[e];
       }
     }
   };
 
-  float m_run[kQT], l_run[kQT];
-  f32x4 acc[kQT][kDT];
+  float m_run = -INFINITY, l_run = 0.0f;
+  f32x4 acc[kDT];
 #pragma unroll
-  for (int u = 0; u < kQT; u++) {
-    m_run[u] = -INFINITY;
-    l_run[u] = 0.0f;
+  for (int dt = 0; dt < kDT; dt++) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // this wave's part of the tile in LDS, positions p0 ..
+  auto attend = [&](int p0) __attribute__((always_inline)) {
+    f32x4 s[2];
 #pragma unroll
-    for (int dt = 0; dt < kDT; dt++) acc[u][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+    for (int tt = 0; tt < 2; tt++) s[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < kKK; kk++)
+#pragma unroll
+      for (int tt = 0; tt < 2; tt++) {
+        const f16x8 kf = *reinterpret_cast<const f16x8 *>(
+            &ks[(32 * kh + 16 * tt + r) * kKRow + 32 * kk + 8 * grp]);
+#pragma unroll
+        for (int part = 0; part < kParts; part++)
+          s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[part][kk], s[tt], 0, 0, 0);
+      }
+    if (p0 + 31 > qlo) {
+      const int seen = qpos - p0 - 4 * grp;  // positions up to this one
+#pragma unroll
+      for (int tt = 0; tt < 2; tt++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          if (16 * tt + e > seen) s[tt][e] = -INFINITY;
+    }
+    float mx = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
+                     fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (__any(mx > m_run)) {
+      const float m_new = fmaxf(m_run, mx);
+      const float corr = m_run == m_new ? 1.0f : exp_neg(m_run - m_new);
+      m_run = m_new;
+      l_run *= corr;
+#pragma unroll
+      for (int dt = 0; dt < kDT; dt++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[dt][e] *= corr;
+    }
+    // (-inf while this part has shown the token nothing)
+    const float m = m_run == -INFINITY ? 0.0f : m_run;
+    f16x8 p[kParts];
+    float ls = 0.0f;
+#pragma unroll
+    for (int tt = 0; tt < 2; tt++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        // (one fp16 holds 11 bits of P: the plain exp2 is far below that)
+        const float x = s[tt][e] - m;
+        const float pr = kSplit ? exp_neg(x) : __builtin_amdgcn_exp2f(x * 1.44269504f);
+        const _Float16 hi = (_Float16)pr;
+        p[0][tt * 4 + e] = hi;
+        if (kSplit) {
+          p[kParts - 1][tt * 4 + e] = (_Float16)(pr - (float)hi);
+          ls += pr;
+        } else {
+          ls += (float)hi;
+        }
+      }
+    l_run += ls;  // this lane's positions; the groups are summed at the end
+#pragma unroll
+    for (int dt = 0; dt < kDT; dt++) {
+      const _Float16 *vrow = &vs[(16 * dt + r) * kVRow + 32 * kh + 4 * grp];
+      const f16x4 v0 = *reinterpret_cast<const f16x4 *>(vrow);
+      const f16x4 v1 = *reinterpret_cast<const f16x4 *>(vrow + 16);
+      const f16x8 vf = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+      for (int part = 0; part < kParts; part++)
+        acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, p[part], acc[dt], 0, 0, 0);
+    }
+  };
   load(0);
   for (int pt = 0; pt < kend; pt += kKeys) {
     lds_barrier();  // the previous tile's reads are done
     store(pt);
     lds_barrier();
     if (pt + kKeys < kend) load(pt + kKeys);
-
-    f32x4 s[kQT][4];
-#pragma unroll
-    for (int u = 0; u < kQT; u++)
-#pragma unroll
-      for (int tt = 0; tt < 4; tt++) s[u][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int tt = 0; tt < 4; tt++)
-#pragma unroll
-      for (int kk = 0; kk < kKK; kk++) {
-        const f16x8 kf =
-            *reinterpret_cast<const f16x8 *>(&ks[(16 * tt + r) * kKRow + 32 * kk + 8 * grp]);
-#pragma unroll
-        for (int u = 0; u < kQT; u++)
-#pragma unroll
-          for (int part = 0; part < kParts; part++)
-            s[u][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[u][part][kk], s[u][tt], 0, 0, 0);
-      }
-
-    f16x8 p[kQT][kParts][2];
-#pragma unroll
-    for (int u = 0; u < kQT; u++) {
-      float mx = -INFINITY;
-#pragma unroll
-      for (int tt = 0; tt < 4; tt++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          if (pt + 16 * tt + 4 * grp + e > qpos[u]) s[u][tt][e] = -INFINITY;
-          mx = fmaxf(mx, s[u][tt][e]);
-        }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float m_new = fmaxf(m_run[u], mx);  // finite: position 0 is always visible
-      const float corr = expf(m_run[u] - m_new);
-      m_run[u] = m_new;
-      float ls = 0.0f;
-#pragma unroll
-      for (int tt = 0; tt < 4; tt++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const float pr = expf(s[u][tt][e] - m_new);
-          const _Float16 hi = (_Float16)pr;
-          p[u][0][tt >> 1][(tt & 1) * 4 + e] = hi;
-          if (kSplit) {
-            p[u][kParts - 1][tt >> 1][(tt & 1) * 4 + e] = (_Float16)(pr - (float)hi);
-            ls += pr;
-          } else {
-            ls += (float)hi;
-          }
-        }
-      l_run[u] = l_run[u] * corr + ls;  // this lane's positions; the groups are summed at the end
-#pragma unroll
-      for (int dt = 0; dt < kDT; dt++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) acc[u][dt][e] *= corr;
-    }
-#pragma unroll
-    for (int dt = 0; dt < kDT; dt++)
-#pragma unroll
-      for (int sl = 0; sl < 2; sl++) {
-        const _Float16 *vrow = &vs[(16 * dt + r) * kVRow + 32 * sl + 4 * grp];
-        const f16x4 v0 = *reinterpret_cast<const f16x4 *>(vrow);
-        const f16x4 v1 = *reinterpret_cast<const f16x4 *>(vrow + 16);
-        const f16x8 vf = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
-#pragma unroll
-        for (int u = 0; u < kQT; u++)
-#pragma unroll
-          for (int part = 0; part < kParts; part++)
-            acc[u][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, p[u][part][sl], acc[u][dt], 0, 0, 0);
-      }
+    if (pt + 32 * kh <= qhi) attend(pt + 32 * kh);
   }
 
+  float l = l_run;
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  lds_barrier();  // the last tile's reads are done
 #pragma unroll
-  for (int u = 0; u < kQT; u++) {
-    float l = l_run[u];
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
-    if (q0 + (wave * kQT + u) * 16 + r < a.T) {
+  for (int dt = 0; dt < kDT; dt++) lds.acc[kh][wave][dt][lane] = acc[dt];
+  stat[kh][wave][0][lane] = m_run;
+  stat[kh][wave][1][lane] = l;
+  lds_barrier();
+  // part kh's wave finishes the kh-th of the dims; position 0 is in part 0, so
+  // the maximum is finite
+  float f[kKP], m = -INFINITY, sum = 0.0f;
 #pragma unroll
-      for (int dt = 0; dt < kDT; dt++)
-        *reinterpret_cast<f16x4 *>(a.attn + qrow[u] + 16 * dt + 4 * grp) =
-            f16x4{(_Float16)(acc[u][dt][0] / l), (_Float16)(acc[u][dt][1] / l),
-                  (_Float16)(acc[u][dt][2] / l), (_Float16)(acc[u][dt][3] / l)};
+  for (int k = 0; k < kKP; k++) m = fmaxf(m, f[k] = stat[k][wave][0][lane]);
+#pragma unroll
+  for (int k = 0; k < kKP; k++) {
+    f[k] = exp_neg(f[k] - m);
+    sum += stat[k][wave][1][lane] * f[k];
+  }
+  if (w0 + r >= a.T) return;
+#pragma unroll
+  for (int dj = 0; dj < kDT / kKP; dj++) {
+    const int dt = kh * (kDT / kKP) + dj;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < kKP; k++) {
+      const f32x4 x = lds.acc[k][wave][dt][lane];
+#pragma unroll
+      for (int e = 0; e < 4; e++) o[e] += x[e] * f[k];
     }
+    f16x4 y;
+#pragma unroll
+    for (int e = 0; e < 4; e++) y[e] = (_Float16)(o[e] / sum);
+    *reinterpret_cast<f16x4 *>(a.attn + qrow + 16 * dt + 4 * grp) = y;
   }
 }
 
@@ -518,7 +604,7 @@ template <int kW, int kEpi, int kMI>
 hipError_t launch_gemm_tile(hipStream_t s, const PrefillGemmArgs &g) {
   const int tiles_m = (g.M + 32 * kMI - 1) / (32 * kMI);
   const int ntiles = tiles_m * (g.N / (32 * kMI)), per_xcd = (ntiles + 7) / 8;
-  prefill_gemm_kernel<kW, kEpi, kMI><<<per_xcd * 8, kT, 0, s>>>(g, tiles_m, ntiles, per_xcd);
+  prefill_gemm_kernel<kW, kEpi, kMI><<<per_xcd * 8, kT * groups_of(kEpi), 0, s>>>(g, tiles_m, ntiles, per_xcd);
   return hipGetLastError();
 }
 
@@ -575,26 +661,16 @@ hipError_t launch_prefill_qkv(hipStream_t s, const PrefillArgs &a, bool qwen, bo
 }
 
 hipError_t launch_prefill_attention(hipStream_t s, const PrefillArgs &a) {
-  // 128 tokens per workgroup where that leaves two workgroups per CU, else 64
-  const bool wide = (long long)((a.T + 127) / 128) * a.heads * a.B >= 512;
-  const int per = wide ? 128 : 64;
-  const dim3 grid((a.T + per - 1) / per, a.heads, a.B);
-#define SH_ATTN(D, VT, SPLIT)                                        \
-  do {                                                               \
-    if (wide)                                                        \
-      prefill_attn_kernel<D, VT, SPLIT, 2><<<grid, kT, 0, s>>>(a);   \
-    else                                                             \
-      prefill_attn_kernel<D, VT, SPLIT, 1><<<grid, kT, 0, s>>>(a);   \
-  } while (0)
+  const int per = attn_tokens(a.d);
+  const dim3 grid(a.heads, (a.T + per - 1) / per, a.B);
   if (a.d == 128 && a.vt_stride)
-    SH_ATTN(128, true, false);
+    prefill_attn_kernel<128, true, false><<<grid, kAttnT, 0, s>>>(a);
   else if (a.d == 128)
-    SH_ATTN(128, false, true);
+    prefill_attn_kernel<128, false, true><<<grid, kAttnT, 0, s>>>(a);
   else if (a.d == 64 && !a.vt_stride)
-    SH_ATTN(64, false, true);
+    prefill_attn_kernel<64, false, true><<<grid, kAttnT, 0, s>>>(a);
   else
     return hipErrorInvalidValue;
-#undef SH_ATTN
   return hipGetLastError();
 }
 

@@ -102,6 +102,24 @@ def test_prompt_pass_after_cached_tokens(ctx, cfg):
             _close(_state(m, 2, total), ref)
 
 
+# the attention's blocks of 32 (head_dim 64: 64) tokens and tiles of 128 (64)
+# positions in four (two) parts: one token past a block, an odd and an even
+# number of blocks, one position past a part and past a tile
+@pytest.mark.parametrize("cfg", [QWEN_SMALL, GPT2_SMALL_TEST], ids=["qwen3", "gpt2"])
+@pytest.mark.parametrize("batch,n", [(2, 34), (1, 97), (1, 130), (2, 162), (1, 258)])
+def test_prompt_attention_block_edges(ctx, cfg, batch, n):
+    prompts = np.random.default_rng(n).integers(0, cfg.vocab, (batch, n))
+    with llm.Model(ctx, cfg.with_(max_positions=300)) as m:
+        m.init_random(seed=7, stddev=0.02)
+        _randomize_small_params(m, 1)
+        m.reset(batch)
+        _stepwise(m, prompts)
+        ref = _state(m, batch, n)
+        m.reset(batch)
+        m.generate(prompts, 1)
+        _close(_state(m, batch, n), ref)
+
+
 def test_prompt_pass_rows_do_not_depend_on_the_batch(ctx):
     # 16 sequences of 300 tokens take the pass in chunks of 256 positions; a
     # sequence alone takes it in one: caches and logits bit for bit the same
