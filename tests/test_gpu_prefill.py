@@ -56,8 +56,8 @@ def _close(got, ref):
 
 
 # 7: the fewest tokens that take the pass; 17, 65, 66: edges of the 16-token
-# q / k / v blocks and the 64-token, 64-position attention tiles; 130, 301:
-# a partial last GEMM tile, several attention tiles
+# q / k / v blocks and the 32- or 64-token attention blocks; 130, 301: a partial
+# last GEMM tile, several attention tiles
 @pytest.mark.parametrize("cfg,layers_kernel", [(QWEN_SMALL, "1"), (QWEN_SMALL, "0"),
                                                (QWEN_SMALL.with_(heads=2, hidden=512), "1"),
                                                (GPT2_SMALL_TEST, "1"),
