@@ -528,7 +528,8 @@ SH_API int sh_llm_next_tokens(sh_llm *model, int32_t *tokens);
 /* prompt[b * prompt_len + i] (host): the prompt's tokens, all but the last in
  * one pass over the layers (short prompts: as steps) and the last as a step,
  * then greedy decoding until `steps` tokens per sequence are produced into
- * out[b * steps + j]. The pass's work buffer (up to ~160 MB at the Qwen3 shape)
+ * out[b * steps + j]. The pass leaves what steps over the same tokens would,
+ * bit for bit. Its work buffer (up to ~160 MB at the Qwen3 shape)
  * is allocated by the first prompt and kept until sh_llm_destroy; without the
  * memory for it the prompt runs as steps. */
 SH_API int sh_llm_generate(sh_llm *model, const int32_t *prompt, int prompt_len, int steps,

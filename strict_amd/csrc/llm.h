@@ -72,6 +72,9 @@ struct AttnArgs {
   int *counters = nullptr;          // [B][kv_heads], zero between launches
   uint16_t *out = nullptr;          // [B][out_ld] fp16 head outputs
   int out_ld = 0;
+  // a prompt's pass (launch_attention_prompt): the rows are tokens, row b of
+  // sequence (row0 + b) / seq_rows
+  int row0 = 0, seq_rows = 1;
 };
 
 struct EmbedArgs {
@@ -265,6 +268,12 @@ hipError_t launch_gemv(hipStream_t s, const GemvArgs &a, int weight_type, int pr
                        int max_grid);
 hipError_t launch_attention(hipStream_t s, const AttnArgs &a, int head_dim, int group, bool qwen,
                             int batch);
+// The same over the token rows of a prompt's pass, a.pos holding each one's
+// position: with append only the new k / v of every row are worked out and
+// written to the caches; without, every row attends over its own context,
+// whose k / v are all in the caches already.
+hipError_t launch_attention_prompt(hipStream_t s, const AttnArgs &a, int head_dim, int group,
+                                   bool qwen, int rows, bool append);
 // The tokens a step embeds, for rows b < B.
 struct StepTokens {
   int B = 0;
@@ -285,16 +294,26 @@ hipError_t launch_embed(hipStream_t s, const EmbedArgs &a, int batch);
 // fp16 out16[b] = norm(x[b]) (pro = kProRms or kProLayer), K <= 4096.
 hipError_t launch_norm_rows(hipStream_t s, const GemvArgs &a, int pro);
 
-// ---- prompts in one pass (prefill.hip) -------------------------------------------
+// ---- prompts in one pass (prefill.hip, prefill_layers.hip) -----------------------
 
-// C = A W^T over M token rows: A fp16 [M][lda], W tiled (N % 64 == 0, K % 128
-// == 0), scales and biases as the GEMV's; epilogues kEpiStore, kEpiResidual
-// (out += ), kEpiSwiGLU (FP8) and kEpiGelu (fp16).
+// Which kernels the model's decode steps run on. A prompt's pass sums in the
+// order of those kernels, operation by operation, so that the caches it
+// leaves are the steps' own bit for bit.
+enum { kStepOps = 0, kStepQwenLayers = 1, kStepGpt2Layers = 2 };
+
+// C = A W^T over M token rows: A fp16 [M][K], in 16-row tiles as fp16 weights
+// are (f16_tiled_offset; a_tiled) or row-major, W tiled (N % 64 == 0, K % 128
+// == 0, FP8: K % 256 == 0), scales and biases as the GEMV's; epilogues
+// kEpiStore, kEpiResidual (out += ), kEpiSwiGLU (FP8) and kEpiGelu (fp16): out
+// [M][out_ld] row-major, out16 [M][out_ld] tiled.
+// inv (kStepQwenLayers, kEpiStore and kEpiSwiGLU): the RMSNorm scale of each
+// token row, applied to the sums.
 struct PrefillGemmArgs {
   const uint8_t *w = nullptr;
-  const float *scale = nullptr, *bias = nullptr;
+  const float *scale = nullptr, *bias = nullptr, *inv = nullptr;
   const uint16_t *a = nullptr;
-  int lda = 0, M = 0, K = 0, N = 0;
+  bool a_tiled = true;
+  int M = 0, K = 0, N = 0;
   float *out = nullptr;
   uint16_t *out16 = nullptr;
   int out_ld = 0;
@@ -307,7 +326,8 @@ struct PrefillArgs {
   const int *lens = nullptr;    // [B] positions cached before the prompt
   int prompt_len = 0, i0 = 0, T = 0, B = 0;
   int H = 0, heads = 0, kv_heads = 0, d = 0, qkv_n = 0, max_pos = 0;
-  int vt_stride = 0;            // positions per V^T cache row; 0: V as [max_pos][d]
+  int splits = 1, chunk = 16;   // the steps' attention splits
+  int vt_stride = 0;            // kStepQwenLayers: positions per V^T cache row
   float eps = 0.0f, scale = 1.0f;
   // embedding
   int *hist = nullptr;
@@ -317,20 +337,36 @@ struct PrefillArgs {
   const uint16_t *head16 = nullptr, *wpe = nullptr;
   const float *inv_freq = nullptr;
   float *rope = nullptr;        // [B * T][d]: cos | sin
+  int *pos = nullptr;           // [B * T]
   float *x = nullptr;           // [B * T][H] residual stream
+  // norms: tiled fp16 rows (kStepQwenLayers: x times the gain, the row's scale in inv)
+  uint16_t *h16 = nullptr;
+  float *inv = nullptr;
   // attention
   const float *qkv = nullptr, *q_norm = nullptr, *k_norm = nullptr;  // qkv [B * T][qkv_n]
-  uint16_t *q = nullptr, *q_lo = nullptr;  // [B * T][heads][d], scaled
+  uint16_t *q = nullptr;        // kStepQwenLayers: [B * T][heads][d], scaled
+  float *smax = nullptr;        // kStepQwenLayers: [B * T][heads][splits] score maxima
   uint16_t *kcache = nullptr, *vcache = nullptr;
-  uint16_t *attn = nullptr;     // [B * T][heads * d] fp16
+  uint16_t *attn = nullptr;     // [B * T][heads * d] fp16, tiled (kStepOps: row-major)
 };
 hipError_t launch_prefill_embed(hipStream_t s, const PrefillArgs &a);
-hipError_t launch_prefill_gemm(hipStream_t s, const PrefillGemmArgs &g, int weight_type, int epi);
+hipError_t launch_prefill_finish(hipStream_t s, int *lens, int B, int n);  // lens[b] += n
+// kStepOps and kStepGpt2Layers
+hipError_t launch_prefill_norm(hipStream_t s, const PrefillArgs &a, const float *gamma,
+                               const float *beta, int form);
+hipError_t launch_prefill_gemm(hipStream_t s, const PrefillGemmArgs &g, int weight_type, int epi,
+                               int form);
+// k and v of a layer appended to the caches as they are (GPT-2)
+hipError_t launch_prefill_append(hipStream_t s, const PrefillArgs &a);
+hipError_t launch_prefill_attention_gpt2(hipStream_t s, const PrefillArgs &a);  // B = 1, d = 64
+// kStepQwenLayers (d = 128, two query heads per KV head)
+hipError_t launch_prefill_norm_layers(hipStream_t s, const PrefillArgs &a, const float *gamma);
+hipError_t launch_prefill_gemm_layers(hipStream_t s, const PrefillGemmArgs &g, int epi);
 // q, k, v of a layer: norms and RoPE, q out, k and v appended to the caches
 // (kv_only: without the query heads).
-hipError_t launch_prefill_qkv(hipStream_t s, const PrefillArgs &a, bool qwen, bool kv_only);
-hipError_t launch_prefill_attention(hipStream_t s, const PrefillArgs &a);
-hipError_t launch_prefill_finish(hipStream_t s, int *lens, int B, int n);  // lens[b] += n
+hipError_t launch_prefill_qkv_layers(hipStream_t s, const PrefillArgs &a, bool kv_only);
+hipError_t launch_prefill_attention_layers(hipStream_t s, const PrefillArgs &a);
+hipError_t prepare_prefill_kernels();  // on the current device, before the launches above
 
 hipError_t launch_quantize_e4m3_tiled(hipStream_t s, const float *w, int N, int K,
                                       int interleave_rows, uint8_t *q, float *scales,

@@ -506,74 +506,86 @@ int setup_gpt2_kernel(sh_llm *m) {
 
 // ---- a prompt's pass -------------------------------------------------------------
 
-// Token rows of one chunk of the pass: enough for full GEMM tiles on every
-// CU; the work buffer is ~40 KB a row at the Qwen3 shape (160 MB).
+// Token rows of one chunk of the pass: enough for GEMM tiles on every CU; the
+// work buffer is ~40 KB a row at the Qwen3 shape (160 MB).
 constexpr int kPrefillRows = 4096;
-// Fewest tokens a sequence brings for the pass to be taken: it takes ~2.2 ms
-// at the Qwen3 shape and ~0.85 ms at GPT-2 small's however few tokens there
-// are, a step 0.40 and 0.145 ms at batch 1 (more at larger batches, 1.3 ms at
-// Qwen3's 16): 6 tokens are where batch 1 breaks even. The rule leaves the
-// batch out, so that a sequence takes the same path in any batch.
-constexpr int kPrefillMinTokens = 6;
+// Fewest tokens a sequence brings for the pass to be taken: it takes 1.49 ms at
+// the Qwen3 shape and 0.61 ms at GPT-2 small's however few tokens there are, a
+// step 0.39 and 0.14 ms at batch 1 (4 tokens are where that breaks even) and
+// more at larger batches (1.3 and 0.76 ms at 16).
+constexpr int kPrefillMinTokens = 4;
+
+// Bytes of the per-op attention's partials in flight at once (rows with
+// several splits go through the kernel in slices).
+constexpr size_t kPrefillPartBytes = (size_t)64 << 20;
+
+// The kernels a prompt's pass takes the place of: the ones a step would run.
+int step_form(const sh_llm *m) {
+  if (m->layers_kernel) return kStepQwenLayers;
+  return m->gpt2_kernel && m->batch == 1 ? kStepGpt2Layers : kStepOps;
+}
+
+// Token rows per slice of the per-op attention.
+int prefill_slice(const sh_llm *m, int rows) {
+  if (m->splits <= 1) return rows;
+  const size_t row = (size_t)m->cfg.heads * m->splits * (m->cfg.head_dim + 2) * 4;
+  return (int)std::max<size_t>(1, std::min<size_t>(rows, kPrefillPartBytes / row));
+}
 
 // The parts of the work buffer for `rows` token rows, each at a multiple of
 // 256 bytes; returns the whole size (base NULL: only that).
-size_t prefill_layout(const sh_llm *m, int rows, uint8_t *base, PrefillArgs *a, uint16_t **h16,
-                      float **qkv, uint16_t **act) {
+size_t prefill_layout(const sh_llm *m, int rows, uint8_t *base, PrefillArgs *a, float **qkv,
+                      uint16_t **act, float **partials) {
   const sh_llm_config &c = m->cfg;
-  const size_t R = (size_t)rows, HD = (size_t)c.heads * c.head_dim;
+  const size_t R = (size_t)(rows + 15) / 16 * 16, HD = (size_t)c.heads * c.head_dim;  // (whole tiles)
   size_t at = 0;
   auto part = [&](size_t bytes) {
     void *p = base ? base + at : nullptr;
     at += (bytes + 255) & ~(size_t)255;
     return p;
   };
-  int *tokens = static_cast<int *>(part((size_t)c.max_batch * c.max_positions * 4));
-  float *x = static_cast<float *>(part(R * c.hidden * 4));
-  *h16 = static_cast<uint16_t *>(part(R * c.hidden * 2));
+  a->tokens = static_cast<int *>(part((size_t)c.max_batch * c.max_positions * 4));
+  a->pos = static_cast<int *>(part(R * 4));
+  a->x = static_cast<float *>(part(R * c.hidden * 4));
+  a->h16 = static_cast<uint16_t *>(part(R * c.hidden * 2));
   *qkv = static_cast<float *>(part(R * m->qkv_n * 4));
-  uint16_t *q = static_cast<uint16_t *>(part(R * HD * 2));
-  // the decode-layers kernel's models keep q in one fp16, the others in two
-  uint16_t *q_lo = m->layers_kernel ? nullptr : static_cast<uint16_t *>(part(R * HD * 2));
-  uint16_t *attn = static_cast<uint16_t *>(part(R * HD * 2));
+  a->q = m->layers_kernel ? static_cast<uint16_t *>(part(R * HD * 2)) : nullptr;
+  a->inv = m->layers_kernel ? static_cast<float *>(part(R * 4)) : nullptr;
+  a->smax = m->layers_kernel ? static_cast<float *>(part(R * c.heads * m->la.splits * 4)) : nullptr;
+  a->attn = static_cast<uint16_t *>(part(R * HD * 2));
   *act = static_cast<uint16_t *>(part(R * c.intermediate * 2));
-  float *rope = m->qwen ? static_cast<float *>(part(R * c.head_dim * 4)) : nullptr;
-  if (a) {
-    a->tokens = tokens;
-    a->x = x;
-    a->qkv = *qkv;
-    a->q = q;
-    a->q_lo = q_lo;
-    a->attn = attn;
-    a->rope = rope;
-  }
+  a->rope = m->qwen ? static_cast<float *>(part(R * c.head_dim * 4)) : nullptr;
+  // (per-op models: the partials of a slice of the rows)
+  *partials = !m->layers_kernel && m->splits > 1
+                  ? static_cast<float *>(part((size_t)prefill_slice(m, rows) * c.heads * m->splits * (c.head_dim + 2) * 4))
+                  : nullptr;
+  a->qkv = *qkv;
   return at;
 }
 
 // Runs tokens 0 .. n - 1 of every sequence's prompt (host, [batch][prompt_len],
 // checked against the vocabulary) through the layers in one pass: the KV
-// caches, lengths and history end up as after n steps. The last layer stops
-// at its k and v, which are all that a later step reads of these tokens. *ran
-// is false, and nothing was enqueued, when there is no memory for the work
-// buffer.
+// caches, lengths and history end up as after n steps, bit for bit. The last
+// layer stops at its k and v, which are all that a later step reads of these
+// tokens. *ran is false, and nothing was enqueued, when there is no memory for
+// the work buffer.
 int prefill(sh_llm *m, const int32_t *prompt, int prompt_len, int n, bool *ran) {
   const sh_llm_config &c = m->cfg;
   hipStream_t s = stream_of(m->ctx);
   const int B = m->batch, H = c.hidden, HD = c.heads * c.head_dim;
   const int chunk = std::min(n, std::max(1, kPrefillRows / B));
-  const int pro = m->qwen ? kProRms : kProLayer;
+  const int form = step_form(m);
   *ran = false;
   PrefillArgs a;
-  uint16_t *h16 = nullptr, *act = nullptr;
-  float *qkv = nullptr;
+  uint16_t *act = nullptr;
+  float *qkv = nullptr, *partials = nullptr;
   if (m->prefill_rows < B * chunk) {
     SH_HIP_TRY(hipStreamSynchronize(s));  // an earlier prompt's pass may still use it
     if (m->prefill_buf) (void)hipFree(m->prefill_buf);
     m->prefill_buf = nullptr;
     m->prefill_rows = 0;
     const int rows = std::min(kPrefillRows, (B * chunk + 255) / 256 * 256);
-    const hipError_t e =
-        hipMalloc(&m->prefill_buf, prefill_layout(m, rows, nullptr, nullptr, &h16, &qkv, &act));
+    const hipError_t e = hipMalloc(&m->prefill_buf, prefill_layout(m, rows, nullptr, &a, &qkv, &act, &partials));
     if (e != hipSuccess) {
       m->prefill_buf = nullptr;
       (void)hipGetLastError();
@@ -581,7 +593,7 @@ int prefill(sh_llm *m, const int32_t *prompt, int prompt_len, int n, bool *ran) 
     }
     m->prefill_rows = rows;
   }
-  prefill_layout(m, m->prefill_rows, static_cast<uint8_t *>(m->prefill_buf), &a, &h16, &qkv, &act);
+  prefill_layout(m, m->prefill_rows, static_cast<uint8_t *>(m->prefill_buf), &a, &qkv, &act, &partials);
   *ran = true;
   SH_HIP_TRY(hipMemcpyAsync(const_cast<int *>(a.tokens), prompt, (size_t)B * prompt_len * 4,
                             hipMemcpyHostToDevice, s));
@@ -595,7 +607,9 @@ int prefill(sh_llm *m, const int32_t *prompt, int prompt_len, int n, bool *ran) 
   a.d = c.head_dim;
   a.qkv_n = m->qkv_n;
   a.max_pos = c.max_positions;
-  a.vt_stride = m->layers_kernel ? m->la.vt_stride : 0;
+  a.splits = form == kStepQwenLayers ? m->la.splits : form == kStepGpt2Layers ? kGpt2Splits : m->splits;
+  a.chunk = form == kStepQwenLayers ? m->la.chunk : form == kStepGpt2Layers ? m->ga.chunk : m->chunk;
+  a.vt_stride = form == kStepQwenLayers ? m->la.vt_stride : 0;
   a.eps = c.norm_eps;
   a.scale = 1.0f / std::sqrt((float)c.head_dim);
   a.hist = m->hist;
@@ -611,34 +625,59 @@ int prefill(sh_llm *m, const int32_t *prompt, int prompt_len, int n, bool *ran) 
     a.T = std::min(chunk, n - i0);
     const int M = B * a.T;
     auto norm = [&](const float *gamma, const float *beta) {
-      GemvArgs g;
-      g.x = a.x;
-      g.x_ld = H;
-      g.gamma = gamma;
-      g.beta = beta;
-      g.eps = c.norm_eps;
-      g.B = M;
-      g.K = H;
-      g.out16 = h16;
-      g.out_ld = H;
-      return launch_norm_rows(s, g, pro);
+      return form == kStepQwenLayers ? launch_prefill_norm_layers(s, a, gamma)
+                                     : launch_prefill_norm(s, a, gamma, beta, form);
     };
-    // rows n0 .. of `l` from A, as the step's GEMVs take them
+    // rows n0 .. of `l` from the fp16 rows `in`
     auto linear = [&](const Linear &l, const uint16_t *in, int n0, float *out, uint16_t *out16,
                       int out_ld, int epi) {
       PrefillGemmArgs g;
       g.w = l.w + (size_t)n0 * l.K * (m->wtype == kWeightFp8 ? 1 : 2);
       g.scale = l.scale ? l.scale + n0 : nullptr;
       g.bias = l.bias ? l.bias + n0 : nullptr;
+      g.inv = a.inv;
       g.a = in;
-      g.lda = l.K;
+      g.a_tiled = form != kStepOps || in != a.attn;
       g.M = M;
       g.K = l.K;
       g.N = l.N - n0;
       g.out = out ? out + n0 : nullptr;
       g.out16 = out16;
       g.out_ld = out_ld;
-      return launch_prefill_gemm(s, g, m->wtype, epi);
+      return form == kStepQwenLayers ? launch_prefill_gemm_layers(s, g, epi)
+                                     : launch_prefill_gemm(s, g, m->wtype, epi, form);
+    };
+    // the per-op step's attention kernel over token rows, in slices whose
+    // partials fit
+    auto attention_ops = [&](const Layer &L, bool append) {
+      AttnArgs t;
+      t.qkv_ld = m->qkv_n;
+      t.kcache = L.kcache;
+      t.vcache = L.vcache;
+      t.max_pos = c.max_positions;
+      t.q_norm = L.q_norm;
+      t.k_norm = L.k_norm;
+      t.eps = c.norm_eps;
+      t.scale = a.scale;
+      t.heads = c.heads;
+      t.kv_heads = c.kv_heads;
+      t.splits = m->splits;
+      t.chunk = m->chunk;
+      t.part = partials;
+      t.out_ld = HD;
+      t.seq_rows = a.T;
+      const int slice = prefill_slice(m, M);
+      for (int r0 = 0; r0 < M; r0 += slice) {
+        t.row0 = r0;
+        t.qkv = qkv + (size_t)r0 * m->qkv_n;
+        t.pos = a.pos + r0;
+        t.rope = a.rope ? a.rope + (size_t)r0 * c.head_dim : nullptr;
+        t.out = a.attn + (size_t)r0 * HD;
+        const hipError_t e = launch_attention_prompt(s, t, c.head_dim, c.heads / c.kv_heads, m->qwen,
+                                                     std::min(slice, M - r0), append);
+        if (e != hipSuccess) return e;
+      }
+      return hipSuccess;
     };
     SH_HIP_TRY(launch_prefill_embed(s, a));
     for (size_t li = 0; li < m->layers.size(); li++) {
@@ -649,13 +688,23 @@ int prefill(sh_llm *m, const int32_t *prompt, int prompt_len, int n, bool *ran) 
       a.kcache = L.kcache;
       a.vcache = L.vcache;
       SH_HIP_TRY(norm(L.norm1_g, L.norm1_b));
-      SH_HIP_TRY(linear(L.qkv, h16, last ? HD : 0, qkv, nullptr, m->qkv_n, kEpiStore));
-      SH_HIP_TRY(launch_prefill_qkv(s, a, m->qwen, last));
-      if (last) break;
-      SH_HIP_TRY(launch_prefill_attention(s, a));
+      SH_HIP_TRY(linear(L.qkv, a.h16, last ? HD : 0, qkv, nullptr, m->qkv_n, kEpiStore));
+      if (form == kStepQwenLayers) {
+        SH_HIP_TRY(launch_prefill_qkv_layers(s, a, last));
+        if (last) break;
+        SH_HIP_TRY(launch_prefill_attention_layers(s, a));
+      } else if (!m->qwen) {
+        SH_HIP_TRY(launch_prefill_append(s, a));
+        if (last) break;
+        SH_HIP_TRY(form == kStepGpt2Layers ? launch_prefill_attention_gpt2(s, a) : attention_ops(L, false));
+      } else {
+        SH_HIP_TRY(attention_ops(L, true));
+        if (last) break;
+        SH_HIP_TRY(attention_ops(L, false));
+      }
       SH_HIP_TRY(linear(L.o, a.attn, 0, a.x, nullptr, H, kEpiResidual));
       SH_HIP_TRY(norm(L.norm2_g, L.norm2_b));
-      SH_HIP_TRY(linear(L.up, h16, 0, nullptr, act, c.intermediate, m->qwen ? kEpiSwiGLU : kEpiGelu));
+      SH_HIP_TRY(linear(L.up, a.h16, 0, nullptr, act, c.intermediate, m->qwen ? kEpiSwiGLU : kEpiGelu));
       SH_HIP_TRY(linear(L.down, act, 0, a.x, nullptr, H, kEpiResidual));
     }
   }
@@ -849,6 +898,7 @@ SH_API int sh_llm_create(sh_ctx *ctx, const sh_llm_config *config, sh_llm **out)
   }
   if ((rc = fill(m, m->final_g, H, 1.0f))) return cleanup(rc);
   hipError_t e = prepare_gemv_kernels();
+  if (e == hipSuccess) e = prepare_prefill_kernels();
   if (e == hipSuccess) e = hipStreamSynchronize(stream_of(ctx));
   if (e != hipSuccess) return cleanup(hip_fail(e, "preparing the model"));
   if ((rc = setup_layers_kernel(m)) != SH_OK) return cleanup(rc);

@@ -23,6 +23,23 @@ __device__ __forceinline__ float f16_bits_to_f32(uint16_t h) {
   return (float)__builtin_bit_cast(_Float16, h);
 }
 
+// a * b rounded once, to fp16: what a product that is only used as fp16 becomes
+// in the step kernels (v_fma_mixlo_f16). The prompt pass, which computes the
+// same values, names it, so that neither depends on what surrounds it.
+__device__ __forceinline__ _Float16 f16_product(float a, float b) {
+  uint32_t r = 0;
+  asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "+v"(r) : "v"(a), "v"(b));
+  return __builtin_bit_cast(_Float16, (uint16_t)r);
+}
+
+// x, a rounded fp32 value, to fp16 (never one rounding with the operation
+// that made it).
+__device__ __forceinline__ _Float16 f16_of_f32(float x) {
+  uint32_t r;
+  asm("v_cvt_f16_f32 %0, %1" : "=v"(r) : "v"(x));
+  return __builtin_bit_cast(_Float16, (uint16_t)r);
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
@@ -136,6 +153,12 @@ __device__ __forceinline__ size_t f16_tiled_offset(int n, int k, int K) {
 __device__ __forceinline__ float gelu_tanh(float x) {
   const float c = 0.7978845608028654f;  // sqrt(2 / pi)
   return 0.5f * x * (1.0f + tanhf(c * (x + 0.044715f * x * x * x)));
+}
+
+// gelu_tanh(x) as fp16, its last product rounded once.
+__device__ __forceinline__ _Float16 gelu_tanh_f16(float x) {
+  const float c = 0.7978845608028654f;
+  return f16_product(0.5f * x, 1.0f + tanhf(c * (x + 0.044715f * x * x * x)));
 }
 
 // Eight fp16 MFMA B-operand values from 8 E4M3 bytes (two dwords), exact.

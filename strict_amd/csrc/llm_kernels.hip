@@ -479,7 +479,11 @@ __global__ __launch_bounds__(kThreads, kL <= 4 ? 4 : 2) void gemv_regs_kernel(co
 // Lane layout: kLPP = d/8 lanes per position, each holding 8 dims (16 bytes
 // of fp16 K or V); a wave covers kPPW positions per load. Every K (then V)
 // load of a thread for up to kBatch positions is issued before any is used.
-template <int kD, int kG, bool kQwen>
+//
+// kMode kAttnAppend / kAttnPrompt: the same over the token rows of a prompt's
+// pass (launch_attention_prompt), so that a token's arithmetic is a step's.
+enum { kAttnStep = 0, kAttnAppend = 1, kAttnPrompt = 2 };
+template <int kD, int kG, bool kQwen, int kMode>
 __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const AttnArgs a) {
   constexpr int kLPP = kD / 8;        // lanes per position (8 dims each)
   constexpr int kPPW = 64 / kLPP;     // positions per wave step
@@ -502,7 +506,8 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const AttnArgs a)
   const int p0 = s * chunk;
   if (p0 >= a.max_pos) return;
   const float *qkv = a.qkv + (size_t)b * a.qkv_ld;
-  const size_t cache_base = ((size_t)b * a.kv_heads + kvh) * (size_t)a.max_pos * kD;
+  const int seq = kMode == kAttnStep ? b : (a.row0 + b) / a.seq_rows;
+  const size_t cache_base = ((size_t)seq * a.kv_heads + kvh) * (size_t)a.max_pos * kD;
   const int seg = lane % kLPP, sub = lane / kLPP;
   const uint16_t *kbase = a.kcache + cache_base + seg * 8;
   const uint16_t *vbase = a.vcache + cache_base + seg * 8;
@@ -548,6 +553,7 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const AttnArgs a)
   const int p1 = min(L, p0 + chunk), np = p1 - p0;
   const int pos = L - 1;
   const bool holds_new = p1 == L;
+  if (kMode == kAttnAppend && !holds_new) return;
   const bool kv_thread = holds_new && may_hold_new;
   if (!q_thread) qv = 0.0f;
   if (!kv_thread) kv = vv = 0.0f;
@@ -591,12 +597,16 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const AttnArgs a)
     }
     if (q_thread) qs[gq][iq] = qv * a.scale;
     if (kv_thread) {
-      const _Float16 k16 = (_Float16)kv, v16 = (_Float16)vv;
+      // (a step has kv in fp32 for other uses)
+      const _Float16 k16 = kMode == kAttnAppend ? f16_of_f32(kv) : (_Float16)kv, v16 = (_Float16)vv;
       knew[iq] = k16;
       vnew[iq] = v16;
-      a.kcache[cache_base + (size_t)pos * kD + iq] = __builtin_bit_cast(uint16_t, k16);
-      a.vcache[cache_base + (size_t)pos * kD + iq] = __builtin_bit_cast(uint16_t, v16);
+      if (kMode != kAttnPrompt) {
+        a.kcache[cache_base + (size_t)pos * kD + iq] = __builtin_bit_cast(uint16_t, k16);
+        a.vcache[cache_base + (size_t)pos * kD + iq] = __builtin_bit_cast(uint16_t, v16);
+      }
     }
+    if (kMode == kAttnAppend) return;
     __syncthreads();
   }
 
@@ -1017,9 +1027,6 @@ hipError_t launch_gemv(hipStream_t s, const GemvArgs &a_in, int weight_type, int
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_attention_partials(hipStream_t s, const AttnArgs &a, int head_dim, int group,
-                                     bool qwen, dim3 grid);
-
 hipError_t prepare_gemv_kernels() {
   hipError_t e = hipSuccess;
 #define SH_ALLOW(W, P, E) \
@@ -1029,32 +1036,45 @@ hipError_t prepare_gemv_kernels() {
   return e;
 }
 
-hipError_t launch_attention(hipStream_t s, const AttnArgs &a, int head_dim, int group, bool qwen,
-                            int batch) {
-  dim3 grid(a.splits, a.kv_heads, batch);
-  hipError_t e = launch_attention_partials(s, a, head_dim, group, qwen, grid);
-  if (e != hipSuccess || a.splits == 1) return e;
-  dim3 mgrid(a.heads, batch);
-  if (head_dim == 128)
-    attn_merge_kernel<128><<<mgrid, 128, 0, s>>>(a);
-  else
-    attn_merge_kernel<64><<<mgrid, 64, 0, s>>>(a);
-  return hipGetLastError();
-}
-
-hipError_t launch_attention_partials(hipStream_t s, const AttnArgs &a, int head_dim, int group,
-                                     bool qwen, dim3 grid) {
+template <int kMode>
+static hipError_t launch_attention_partials(hipStream_t s, const AttnArgs &a, int head_dim, int group,
+                                            bool qwen, dim3 grid) {
   if (head_dim == 128 && group == 2 && qwen)
-    attn_decode_kernel<128, 2, true><<<grid, kThreads, 0, s>>>(a);
+    attn_decode_kernel<128, 2, true, kMode><<<grid, kThreads, 0, s>>>(a);
   else if (head_dim == 128 && group == 1 && qwen)
-    attn_decode_kernel<128, 1, true><<<grid, kThreads, 0, s>>>(a);
+    attn_decode_kernel<128, 1, true, kMode><<<grid, kThreads, 0, s>>>(a);
   else if (head_dim == 64 && group == 1 && !qwen)
-    attn_decode_kernel<64, 1, false><<<grid, kThreads, 0, s>>>(a);
+    attn_decode_kernel<64, 1, false, kMode><<<grid, kThreads, 0, s>>>(a);
   else if (head_dim == 128 && group == 1 && !qwen)
-    attn_decode_kernel<128, 1, false><<<grid, kThreads, 0, s>>>(a);
+    attn_decode_kernel<128, 1, false, kMode><<<grid, kThreads, 0, s>>>(a);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();
+}
+
+static hipError_t launch_attention_merge(hipStream_t s, const AttnArgs &a, int head_dim, int rows) {
+  if (a.splits == 1) return hipSuccess;
+  const dim3 grid(a.heads, rows);
+  if (head_dim == 128)
+    attn_merge_kernel<128><<<grid, 128, 0, s>>>(a);
+  else
+    attn_merge_kernel<64><<<grid, 64, 0, s>>>(a);
+  return hipGetLastError();
+}
+
+hipError_t launch_attention(hipStream_t s, const AttnArgs &a, int head_dim, int group, bool qwen,
+                            int batch) {
+  const hipError_t e = launch_attention_partials<kAttnStep>(s, a, head_dim, group, qwen,
+                                                            dim3(a.splits, a.kv_heads, batch));
+  return e != hipSuccess ? e : launch_attention_merge(s, a, head_dim, batch);
+}
+
+hipError_t launch_attention_prompt(hipStream_t s, const AttnArgs &a, int head_dim, int group,
+                                   bool qwen, int rows, bool append) {
+  const dim3 grid(a.splits, a.kv_heads, rows);
+  if (append) return launch_attention_partials<kAttnAppend>(s, a, head_dim, group, qwen, grid);
+  const hipError_t e = launch_attention_partials<kAttnPrompt>(s, a, head_dim, group, qwen, grid);
+  return e != hipSuccess ? e : launch_attention_merge(s, a, head_dim, rows);
 }
 
 hipError_t launch_norm_rows(hipStream_t s, const GemvArgs &a, int pro) {
