@@ -421,6 +421,88 @@ struct AttnOpArgs {
 template <int kD>
 constexpr int kAttnTile = 8 * 256 * 8 / kD;
 
+constexpr float kPScale = 16384.0f;  // of P, and so of a partial's V sums and sum
+
+// The result of a split for value i (head, dim) of the G heads from h0: its
+// partial or, where the split is the whole row, the output.
+template <int kD>
+__device__ __forceinline__ void attn_store(const AttnOpArgs &a, int b, int h0, int s, int i, float sum,
+                                           float m, float l) {
+  if (a.splits == 1) {
+    a.out[((size_t)b * a.heads + h0) * kD + i] = sum / l;
+    return;
+  }
+  float *pp = a.part + (((size_t)b * a.heads + h0 + i / kD) * a.splits + s) * (size_t)(kD + 2);
+  pp[i % kD] = sum;
+  if (i % kD == 0) {
+    pp[kD] = m;
+    pp[kD + 1] = l;
+  }
+}
+
+// Positions [p0, p1) in fp32 throughout, 64 at a time: a wave scores a head
+// (lane: position), a thread sums V for (head, dim) pairs t, t + kT, ... Slow,
+// for splits whose sums in two fp16 are not finite: infinities and NaN in q, K
+// or V. A score of -inf has no weight.
+struct AttnFp32 {
+  float p[kMaxGroup][64], corr[kMaxGroup], m[kMaxGroup], l[kMaxGroup];
+};
+template <int kD>
+__device__ __forceinline__ void attn_fp32(const AttnOpArgs &a, int b, int kvh, int s, int p0,
+                                                    int p1, AttnFp32 &lds) {
+  constexpr int kAcc = kMaxGroup * kD / kT;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, G = a.heads / a.kv_heads, h0 = kvh * G;
+  const size_t row0 = ((size_t)b * a.kv_heads + kvh) * (size_t)a.max_pos;
+  const _Float16 *kb = reinterpret_cast<const _Float16 *>(a.k) + row0 * kD;
+  const _Float16 *vb = reinterpret_cast<const _Float16 *>(a.v) + row0 * kD;
+  if (t < kMaxGroup) {
+    lds.m[t] = -INFINITY;
+    lds.l[t] = 0.0f;
+  }
+  float acc[kAcc];
+#pragma unroll
+  for (int j = 0; j < kAcc; j++) acc[j] = 0.0f;
+  for (int pt = p0; pt < p1; pt += 64) {
+    const int n = min(64, p1 - pt);
+    __syncthreads();  // the last tile's p and corr are read; m and l are set
+    for (int g = wave; g < G; g += 4) {
+      const float *q = a.q + ((size_t)b * a.heads + h0 + g) * kD;
+      const _Float16 *k = kb + (size_t)min(pt + lane, p1 - 1) * kD;
+      float dot = 0.0f;
+#pragma unroll 1
+      for (int c = 0; c < kD; c += 8) {
+        const f16x8 kk = *reinterpret_cast<const f16x8 *>(k + c);
+#pragma unroll
+        for (int e = 0; e < 8; e++) dot = fmaf(q[c + e] * a.scale, (float)kk[e], dot);
+      }
+      const float sc = lane < n ? dot : -INFINITY, old = lds.m[g];
+      const float m = fmaxf(old, wave_max(sc));
+      const float p = sc == -INFINITY ? 0.0f : expf(sc - m), c = old == m ? 1.0f : expf(old - m);
+      const float sum = wave_sum(p);
+      lds.p[g][lane] = p;
+      if (lane == 0) {
+        lds.corr[g] = c;
+        lds.m[g] = m;
+        lds.l[g] = lds.l[g] * c + sum;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kAcc; j++) {
+      const int i = t + kT * j, g = i / kD;
+      if (g >= G) break;
+      float sum = 0.0f;
+      for (int p = 0; p < n; p++) sum = fmaf(lds.p[g][p], (float)vb[(size_t)(pt + p) * kD + i % kD], sum);
+      acc[j] = acc[j] * lds.corr[g] + sum;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kAcc; j++) {
+    const int i = t + kT * j, g = i / kD;
+    if (g < G) attn_store<kD>(a, b, h0, s, i, acc[j] * kPScale, lds.m[g], lds.l[g] * kPScale);
+  }
+}
+
 // grid (splits, kv_heads, B): positions [s * chunk, min((s + 1) * chunk, L)) of
 // row b for the G = heads / kv_heads query heads of KV head kvh, in tiles of
 // kAttnTile positions. The kernel is bound by the K and V bytes, so all of a
@@ -436,9 +518,13 @@ constexpr int kAttnTile = 8 * 256 * 8 / kD;
 //    position 4 g + e of the first block for e < 4, of the second for e >= 4);
 //    V goes through LDS rows as it is and comes back by transposing reads.
 // q and P stay fp32 to 2^-22: q as two fp16 after an exact power-of-two scaling
-// of each head to below 1, P times 2^14 as two fp16. (Error against 64 bits
-// 2.6e-7; the fp32 kernel before it, 64-position tiles staged in LDS with one
-// serial V sum per thread, 4.1e-7.)
+// of each head to below 1, the remainder times 2^12 and on sums of its own (so
+// that values far below their head's largest keep their bits, too: to 2^-37 of
+// it), P times 2^14 as two fp16. (Error against 64 bits 2.3e-7; the fp32 kernel
+// before it, 64-position tiles staged in LDS with one serial V sum per thread,
+// 4.1e-7.)
+// Infinities do not survive that (a part of the other sign, or 0, times one is
+// NaN): a split whose sums are not finite is worked out again in fp32.
 // Measured, both kernels of a call, before and after: 4 rows up to 4,096
 // positions, 16 / 8 heads of 128: 29.7 -> 13.5 us (50 MB, 3.7 TB/s); 16 rows 68.3
 // -> 38.5 (4.7 TB/s); 16 rows of 8,192, 16 / 1 heads 73.7 -> 25.2; 1 row of 384,
@@ -450,11 +536,12 @@ __global__ __launch_bounds__(kT, 3) void attn_op_partials_kernel(const AttnOpArg
   constexpr int kBlocks = kAttnTile<kD> / 4 / 16;  // 16-position blocks per wave and tile
   constexpr int kVLoads = kBlocks * 16 * kD / 8 / 64;
   constexpr int kRow = kD * 2, kChunks = kD / 8;   // a V row in LDS: bytes, 16-byte chunks
-  constexpr float kPScale = 16384.0f;
+  constexpr float kQLow = 4096.0f;
   union Lds {
     uint8_t v[4][kBlocks * 16 * kRow];
     float acc[4][kMaxGroup][kD];
     float q[kMaxGroup][kD];
+    AttnFp32 fp32;
   };
   __shared__ __attribute__((aligned(16))) Lds lds;
   __shared__ __attribute__((aligned(16))) _Float16 qh[2][kMaxGroup][kD + 8];
@@ -532,7 +619,7 @@ __global__ __launch_bounds__(kT, 3) void attn_op_partials_kernel(const AttnOpArg
       const float y = ldexpf(x[e], -ex);
       const _Float16 hi = (_Float16)y;
       qh[0][g][lane + 64 * e] = hi;
-      qh[1][g][lane + 64 * e] = (_Float16)(y - (float)hi);
+      qh[1][g][lane + 64 * e] = (_Float16)((y - (float)hi) * kQLow);
     }
   }
   lds_barrier();
@@ -550,18 +637,23 @@ __global__ __launch_bounds__(kT, 3) void attn_op_partials_kernel(const AttnOpArg
   // used this one's, its V as soon as this one's is in LDS)
   auto tile = [&](int pt, auto more_c) __attribute__((always_inline)) {
     constexpr bool kMore = decltype(more_c)::value;
-    f32x4 sc[kBlocks];
+    f32x4 sc[kBlocks], low[kBlocks];
 #pragma unroll
-    for (int tt = 0; tt < kBlocks; tt++) sc[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int tt = 0; tt < kBlocks; tt++) sc[tt] = low[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kk = 0; kk < kKK; kk++)
 #pragma unroll
       for (int part = 0; part < 2; part++) {
         const f16x8 qf = *reinterpret_cast<const f16x8 *>(&qh[part][min(r16, G - 1)][32 * kk + 8 * grp]);
+        f32x4 (&to)[kBlocks] = part ? low : sc;
 #pragma unroll
         for (int tt = 0; tt < kBlocks; tt++)
-          sc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[tt][kk], qf, sc[tt], 0, 0, 0);
+          to[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[tt][kk], qf, to[tt], 0, 0, 0);
       }
+#pragma unroll
+    for (int tt = 0; tt < kBlocks; tt++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) sc[tt][e] = fmaf(low[tt][e], 1.0f / kQLow, sc[tt][e]);
     if constexpr (kMore) {
       __builtin_amdgcn_sched_barrier(0);
       load_k(pt + kAttnTile<kD>);
@@ -650,7 +742,7 @@ __global__ __launch_bounds__(kT, 3) void attn_op_partials_kernel(const AttnOpArg
   }
   lds_barrier();
   // the split's partial: the four waves' sums against their common maximum
-  const size_t pstride = (size_t)kD + 2;
+  bool finite = true;
   for (int i = t; i < G * kD; i += kT) {
     const int g = i / kD, dd = i % kD;
     float m = stat[0][g][0];
@@ -663,17 +755,10 @@ __global__ __launch_bounds__(kT, 3) void attn_op_partials_kernel(const AttnOpArg
       sum = fmaf(f, lds.acc[w][g][dd], sum);
       l = fmaf(f, stat[w][g][1], l);
     }
-    if (a.splits == 1) {  // the whole row: no merge follows
-      a.out[((size_t)b * a.heads + h0) * kD + i] = sum / l;
-      continue;
-    }
-    float *pp = a.part + (((size_t)b * a.heads + h0 + g) * a.splits + s) * pstride;
-    pp[dd] = sum;
-    if (dd == 0) {
-      pp[kD] = m;
-      pp[kD + 1] = l;
-    }
+    finite = finite && __builtin_fabsf(sum) < INFINITY && l < INFINITY;
+    attn_store<kD>(a, b, h0, s, i, sum, m, l);
   }
+  if (__syncthreads_or(finite ? 0 : 1)) attn_fp32<kD>(a, b, kvh, s, p0, p1, lds.fp32);
 }
 
 // grid (heads, B), 4 kD threads:
@@ -715,9 +800,10 @@ __global__ __launch_bounds__(kD * kMergeParts) void attn_op_merge_kernel(const A
     den *= c;
 #pragma unroll
     for (int u = 0; u < kStep; u++) {
-      const float w = j0 + kMergeParts * u < active ? (m[u] == M ? 1.0f : exp_neg(m[u] - M)) : 0.0f;
-      num = fmaf(w, x[u], num);
-      den = fmaf(w, l[u], den);
+      const bool is = j0 + kMergeParts * u < active;
+      const float w = m[u] == M ? 1.0f : exp_neg(m[u] - M);
+      num = is ? fmaf(w, x[u], num) : num;  // (0 times an infinity is not 0)
+      den = is ? fmaf(w, l[u], den) : den;
     }
   }
   red[part][i] = num;
