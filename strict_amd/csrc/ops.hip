@@ -323,9 +323,8 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
   return r;
 }
 
-constexpr int kArgT = 1024;
-
 // Minimum over the workgroup of kArgT threads, in every thread.
+template <int kArgT>
 __device__ __forceinline__ uint32_t block_min_u32(uint32_t v, uint32_t *red) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) v = min(v, (uint32_t)__shfl_xor((int)v, off, 64));
@@ -339,13 +338,14 @@ __device__ __forceinline__ uint32_t block_min_u32(uint32_t v, uint32_t *red) {
 }
 
 // grid (rows): index[row] = the first position of the row's maximum. One
-// workgroup of 16 waves reads a row, 8 vectors of 4 values in flight per
-// thread, so a row streams at what one CU can load. A vector's maximum is
+// workgroup reads a row, 8 vectors of 4 values in flight per thread, so a row
+// streams at what one CU can load. A vector's maximum is
 // found as floats and only that compared (as its order key) with the thread's
 // best, whose vector is remembered; the position within it is looked up at the
 // end. A row that holds a NaN is scanned again for the first one. 16 rows of
 // 151936: 189 us with 4 waves per row, one value and one 64-bit key comparison
 // at a time; 8.5 us a pass here.
+template <int kArgT>
 __global__ __launch_bounds__(kArgT) void argmax_kernel(const float *__restrict__ x, int n,
                                                        int32_t *__restrict__ index) {
   constexpr int kU = 8;
@@ -356,13 +356,14 @@ __global__ __launch_bounds__(kArgT) void argmax_kernel(const float *__restrict__
   int at = 0;         // first position of the best vector
   bool nan = false;
   // vectors at 0, 4, .., the last one at n - 4 (clamped starts: a vector read
-  // twice changes nothing)
+  // twice changes nothing); unsigned, as a start ahead may pass 2^31
+  const uint32_t un = (uint32_t)n;
   if (n >= 4) {
-    for (int v0 = 4 * t; v0 < n; v0 += 4 * kArgT * kU) {
+    for (uint32_t v0 = 4 * t; v0 < un; v0 += 4 * kArgT * kU) {
       f32x4 v[kU];
 #pragma unroll
       for (int u = 0; u < kU; u++)
-        v[u] = *reinterpret_cast<const f32x4_any *>(xr + min(v0 + 4 * kArgT * u, n - 4));
+        v[u] = *reinterpret_cast<const f32x4_any *>(xr + min(v0 + 4 * kArgT * u, un - 4));
 #pragma unroll
       for (int u = 0; u < kU; u++) {
         nan |= __builtin_isunordered(v[u].x, v[u].y) | __builtin_isunordered(v[u].z, v[u].w);
@@ -370,7 +371,7 @@ __global__ __launch_bounds__(kArgT) void argmax_kernel(const float *__restrict__
         const uint32_t k = order_key(__builtin_bit_cast(uint32_t, m));
         const bool better = k > best;
         best = better ? k : best;
-        at = better ? min(v0 + 4 * kArgT * u, n - 4) : at;
+        at = better ? (int)min(v0 + 4 * kArgT * u, un - 4) : at;
       }
     }
   } else if (t < n) {
@@ -381,23 +382,70 @@ __global__ __launch_bounds__(kArgT) void argmax_kernel(const float *__restrict__
   }
   if (__syncthreads_or(nan)) {
     uint32_t first = 0xffffffffu;
-    for (int i = t; i < n && first == 0xffffffffu; i += kArgT)
-      if (xr[i] != xr[i]) first = (uint32_t)i;
-    first = block_min_u32(first, red);
+    for (uint32_t i = t; i < un && first == 0xffffffffu; i += kArgT)
+      if (xr[i] != xr[i]) first = i;
+    first = block_min_u32<kArgT>(first, red);
     if (t == 0) index[blockIdx.x] = (int32_t)first;
     return;
   }
-  const uint32_t top = ~block_min_u32(~best, red);
+  const uint32_t top = ~block_min_u32<kArgT>(~best, red);
   uint32_t first = 0xffffffffu;
   if (best == top) {
 #pragma unroll
     for (int e = 3; e >= 0; e--) {
-      const int i = min(at + e, n - 1);
+      const int i = (int)min((uint32_t)at + e, un - 1);
       if (order_key(__builtin_bit_cast(uint32_t, xr[i])) == top) first = (uint32_t)i;
     }
   }
-  first = block_min_u32(first, red);
+  first = block_min_u32<kArgT>(first, red);
   if (t == 0) index[blockIdx.x] = (int32_t)first;
+}
+
+// The same for short rows: one wave per row, four rows per workgroup (a row's
+// barriers would take longer than its values). A value's key has its order in
+// the high word and ~index in the low one, so that the largest key is the
+// first of the largest values.
+__global__ __launch_bounds__(kT) void argmax_short_kernel(const float *__restrict__ x, int rows, int n,
+                                                          int32_t *__restrict__ index) {
+  constexpr int kU = 4;
+  const long long row = (long long)blockIdx.x * (kT / 64) + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const float *xr = x + (size_t)row * n;
+  const int lane = threadIdx.x & 63;
+  unsigned long long best = 0;
+  for (int i0 = lane; i0 < n; i0 += 64 * kU) {
+    float v[kU];
+#pragma unroll
+    for (int u = 0; u < kU; u++) v[u] = xr[min(i0 + 64 * u, n - 1)];
+#pragma unroll
+    for (int u = 0; u < kU; u++) {
+      const int i = min(i0 + 64 * u, n - 1);  // (a value read twice changes nothing)
+      const uint32_t k = v[u] != v[u] ? 0xffffffffu : order_key(__builtin_bit_cast(uint32_t, v[u]));
+      const unsigned long long key = ((unsigned long long)k << 32) | (uint32_t)~i;
+      best = key > best ? key : best;
+    }
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    const unsigned long long o = __shfl_xor(best, off, 64);
+    best = o > best ? o : best;
+  }
+  if (lane == 0) index[row] = (int32_t)~(uint32_t)best;
+}
+
+// By the row's length, where the variants crossed: 100,000 rows of 1,000 70 us with
+// a wave each, 237 with 256 threads, of 64 21 and 117 (1,024 threads: 746); 16 rows
+// of 2,048 5.9 and 4.7. 20,000 rows of 8,192 106 us with 256 threads, 345 with 1,024;
+// 16 rows of 32,768 5.5 with 1,024, 22.8 with 256 (one value at a time). A launch
+// takes fewer than 2^32 threads.
+hipError_t launch_argmax(hipStream_t s, const float *x, int rows, int n, int32_t *index) {
+  if (n <= 1024)
+    argmax_short_kernel<<<(unsigned)((rows + 3LL) / 4), kT, 0, s>>>(x, rows, n, index);
+  else if (n <= 8192 || rows >= (1 << 22))
+    argmax_kernel<256><<<rows, 256, 0, s>>>(x, n, index);
+  else
+    argmax_kernel<1024><<<rows, 1024, 0, s>>>(x, n, index);
+  return hipGetLastError();
 }
 
 // ---- decode attention ----------------------------------------------------------
@@ -1030,8 +1078,7 @@ SH_API int sh_argmax_f32(sh_ctx *ctx, const float *x, int rows, int n, int32_t *
   if ((rc = check_range(ctx, x, (size_t)rows * n * 4, "x")) ||
       (rc = check_range(ctx, index, (size_t)rows * 4, "index")))
     return rc;
-  argmax_kernel<<<rows, kArgT, 0, stream_of(ctx)>>>(x, n, index);
-  const hipError_t e = hipGetLastError();
+  const hipError_t e = launch_argmax(stream_of(ctx), x, rows, n, index);
   return e == hipSuccess ? SH_OK : hip_fail(e, "argmax");
 }
 
