@@ -266,12 +266,13 @@ __global__ __launch_bounds__(kT) void rope_kernel(float *__restrict__ x, const i
 // SwiGLU 4.3 -> 4.1 us a launch (19 MB).
 constexpr int kPerThread = 2;
 
-// Vectors of 4 at any alignment, and the n % 4 values after them one each.
+// Vectors of 4 at any alignment, and the n % 4 values after them one each. (One
+// round but for sizes past the grid's limit.)
 template <class Op>
 __device__ __forceinline__ void map4(size_t n, const float *a, const float *b, float *out, Op op) {
   const size_t n4 = n / 4;
-  const size_t base = (size_t)blockIdx.x * kT * kPerThread + threadIdx.x;
-  if (base < n4) {
+  for (size_t base = (size_t)blockIdx.x * kT * kPerThread + threadIdx.x; base < n4;
+       base += (size_t)gridDim.x * kT * kPerThread) {
     f32x4 va[kPerThread], vb[kPerThread];
 #pragma unroll
     for (int u = 0; u < kPerThread; u++) {
@@ -293,8 +294,9 @@ __device__ __forceinline__ void map4(size_t n, const float *a, const float *b, f
   }
 }
 
+// (A launch takes fewer than 2^32 threads.)
 unsigned map4_grid(size_t n) {
-  return (unsigned)std::max<size_t>(1, (n / 4 + kT * kPerThread - 1) / (kT * kPerThread));
+  return (unsigned)std::min<size_t>(std::max<size_t>(1, (n / 4 + kT * kPerThread - 1) / (kT * kPerThread)), 1u << 23);
 }
 
 __global__ __launch_bounds__(kT) void swiglu_kernel(const float *gate, const float *up, float *out,
