@@ -247,7 +247,8 @@ __global__ __launch_bounds__(kT) void rope_kernel(float *__restrict__ x, const i
     x1[u] = xp[at];
     x2[u] = xp[at + half];
   }
-  const float inv_freq = (float)exp2(log2_theta * (-2.0 * (double)i / (double)d));
+  // (theta^0 is 1 for an infinite theta, too)
+  const float inv_freq = i == 0 ? 1.0f : (float)exp2(log2_theta * (-2.0 * (double)i / (double)d));
   const float ang = (float)pos[row] * inv_freq;
   float c, s;
   cos_sin(ang, &c, &s);

@@ -1,7 +1,9 @@
 """The elementwise pieces past the sizes where a grid of one thread per few values
-would need 2^32 threads."""
+would need 2^32 threads, and RoPE at the ends of theta."""
 import numpy as np
 import pytest
+
+import oracle.llm as ollm
 
 pytestmark = pytest.mark.gpu
 
@@ -39,4 +41,24 @@ def test_more_values_than_a_grid_has_threads_for(ctx, op):
         ctx.sync()
         assert np.array_equal(got.to_host(), ref), s
     for b in (x, small, got):
+        b.free()
+
+
+@pytest.mark.parametrize("theta", [np.inf, 3e38, 1.0, 1e-3])
+def test_rope_at_the_ends_of_theta(ctx, theta):
+    # an infinite theta turns the first pair by the position and leaves the others
+    rows, heads, d = 9, 3, 64
+    rng = np.random.default_rng(4)
+    x = rng.normal(0, 1, (rows, heads, d)).astype(np.float32)
+    positions = np.arange(rows, dtype=np.int32)
+    freq = np.array([float(np.float32(theta)) ** (-2.0 * i / d) for i in range(d // 2)]).astype(np.float32)
+    assert freq[0] == 1.0
+    dx, dp = ctx.upload(x), ctx.upload(positions)
+    ctx.rope(dx, dp, rows, heads, d, float(theta))
+    ctx.sync()
+    cos, sin = ollm.rope_tables(freq, positions)
+    ref = ollm.rope(x, cos, sin)
+    # one rounding per product and sum, and of cos and sin
+    assert np.max(np.abs(dx.to_host() - ref)) <= 4 * 2.0 ** -23 * np.max(np.abs(ref))
+    for b in (dx, dp):
         b.free()
