@@ -1122,7 +1122,10 @@ SH_API int sh_llm_step(sh_llm *m, const int32_t *tokens, int want_logits) {
   } else if (m->graph_batch[g] != m->batch || m->graph_keys[g] != key_set(m)) {
     // (a layers kernel's steps at another batch may have moved the step
     // number to the other key set since the capture)
-    if (m->graph[g]) (void)hipGraphExecDestroy(m->graph[g]);
+    if (m->graph[g]) {
+      SH_HIP_TRY(hipStreamSynchronize(s));  // its last launch may still be queued
+      (void)hipGraphExecDestroy(m->graph[g]);
+    }
     m->graph[g] = nullptr;
     m->graph_batch[g] = -1;
     // first step of this batch size runs eagerly, and is captured for replay
