@@ -608,6 +608,48 @@ __global__ __launch_bounds__(kBytesBlock) void blur_bytes_kernel(const BytesArgs
   }
 }
 
+// ---------------------------------------------------------------------------
+// Blur, one pixel per thread reading its 25 taps of each channel through the
+// cache: narrow tall images, whose rows leave most lanes of a byte strip idle.
+// ---------------------------------------------------------------------------
+
+__global__ __launch_bounds__(kBlock) void blur_direct_kernel(const uint8_t *__restrict__ in,
+                                                             uint8_t *__restrict__ out, int width,
+                                                             int height, int channels, int mode,
+                                                             int fuse, int delta,
+                                                             int all_channels) {
+  const long long pix = (long long)blockIdx.x * kBlock + threadIdx.x;
+  if (pix >= (long long)width * height) return;
+  const int x = (int)(pix % width), y = (int)(pix / width);
+  const size_t stride = (size_t)width * channels;
+  for (int ch = 0; ch < channels; ch++) {
+    const bool adjust = fuse && (all_channels || ch < 3);
+    int sum = 0, count = 0;
+    for (int ky = -2; ky <= 2; ky++) {
+      int ny = y + ky;
+      if (mode == SH_BLUR_CONFIG) {
+        ny = min(max(ny, 0), height - 1);
+      } else if (ny < 0 || ny >= height) {
+        continue;
+      }
+      for (int kx = -2; kx <= 2; kx++) {
+        int nx = x + kx;
+        if (mode == SH_BLUR_CONFIG) {
+          nx = min(max(nx, 0), width - 1);
+        } else if (nx < 0 || nx >= width) {
+          continue;
+        }
+        int v = in[(size_t)ny * stride + (size_t)nx * channels + ch];
+        if (adjust) v = min(255, max(0, v + delta));
+        sum += v;
+        count++;
+      }
+    }
+    const int r = mode == SH_BLUR_CONFIG ? (sum + 12) / 25 : sum / count;
+    out[(size_t)y * stride + (size_t)x * channels + ch] = (uint8_t)r;
+  }
+}
+
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 Brightness make_brightness(bool enabled, int channels, int delta, int all_channels) {
@@ -718,11 +760,25 @@ hipError_t launch_blur5_u8(hipStream_t s, const uint8_t *in, uint8_t *out, int w
     launch_blur_stream<kBlurRows>(s, in32, out32, width, height, fuse, delta, all_channels);
     return hipGetLastError();
   }
+  // A byte strip gives a row of a narrow image a wave's time of its own, one pixel
+  // per thread costs by pixels and channels. 1,000,000 rows, config mode: 1 byte a
+  // row 136 us and 11, 8 bytes (2 channels) 111 and 72, 15 bytes (1) 170 and 131,
+  // 16 bytes 112 and 150, 24 bytes 111 and 230; 4 channels: 2 pixels 111 and 92, 3
+  // pixels 117 and 135. Up to some ten thousand rows the strips are one round of
+  // latency: 3 channels at 3,000 rows 5.1 and 8.7 us, at 100,000 22.1 and 12.3. The
+  // images of 2^29 rows, whose strips would need a grid of 2^32 threads, are here.
+  const size_t row_bytes = (size_t)width * channels;
+  if (height >= 32768 && row_bytes < (channels == 4 ? 12 : 16)) {
+    const long long pixels = (long long)width * height;
+    blur_direct_kernel<<<(unsigned)((pixels + kBlock - 1) / kBlock), kBlock, 0, s>>>(
+        in, out, width, height, channels, mode, fuse ? 1 : 0, delta, all_channels);
+    return hipGetLastError();
+  }
   BytesArgs a;
   a.in = in;
   a.out = out;
   a.height = height;
-  a.row_bytes = (size_t)width * channels;
+  a.row_bytes = row_bytes;
   const Brightness br = make_brightness(fuse, channels, delta, all_channels);
   a.mag = br.mag;
   a.mask = br.mask;

@@ -67,3 +67,38 @@ def test_large_images(ctx, w, h, c, mode):
     # 8-row bands (the first two); either side of the RGBA streaming kernel
     img = seeded_bytes(w * h * c, seed=5)
     assert np.array_equal(_gpu(ctx, img, w, h, c, mode), _reference(img, w, h, c, mode))
+
+
+@pytest.mark.parametrize("mode", [strict_amd.BLUR_CONFIG, strict_amd.BLUR_REFERENCE])
+@pytest.mark.parametrize("c", [1, 2, 3, 4])
+def test_narrow_tall_images(ctx, c, mode):
+    # either side of the sizes where a thread takes one pixel
+    for h in (32767, 32768, 32771):
+        for w in sorted({1, 2, 11 // c, 12 // c, 15 // c, 16 // c, 17 // c}):
+            img = seeded_bytes(w * h * c, seed=w * 31 + c)
+            got = _gpu(ctx, img, w, h, c, mode, offset=w % 3)
+            assert np.array_equal(got, _reference(img, w, h, c, mode)), (w, h)
+            got = _gpu(ctx, img, w, h, c, mode, -40, w % 2)
+            assert np.array_equal(got, _reference(img, w, h, c, mode, -40, w % 2 == 1)), (w, h)
+
+
+@pytest.mark.parametrize("mode", [strict_amd.BLUR_CONFIG, strict_amd.BLUR_REFERENCE])
+def test_tallest_image(ctx, mode):
+    # 2^29 rows of one byte: a wave for each 8 rows is a grid of 2^32 threads. The ends
+    # and the middle are those of short images (2 rows beyond their own edges)
+    h, n = 1 << 29, 1 << 24
+    part = seeded_bytes(n, seed=9)
+    src, out = ctx.empty((h,), np.uint8), ctx.upload(np.zeros(h, np.uint8))
+    for s in range(0, h, n):
+        src.view(s, n).copy_from_host(part)
+    ctx.box_blur5(src, out, 1, h, 1, mode)
+    ctx.sync()
+    ref = _reference(part, 1, n, 1, mode)
+    assert np.array_equal(out.view(0, n - 2).to_host(), ref[:-2])
+    assert np.array_equal(out.view(h - n + 2, n - 2).to_host(), ref[2:])
+    joint = np.concatenate([part[-8:], part[:8]])
+    for s in (n, h // 2, h - n):
+        assert np.array_equal(out.view(s - 6, 12).to_host(), _reference(joint, 1, 16, 1, mode)[2:-2])
+        assert np.array_equal(out.view(s + 2, n - 4).to_host(), ref[2:-2]) or s == h - n
+    src.free()
+    out.free()
