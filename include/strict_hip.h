@@ -444,7 +444,8 @@ SH_API int sh_argmax_f32(sh_ctx *ctx, const float *x, int rows, int n, int32_t *
  * [kv_heads][max_positions][head_dim] (the runners' cache layout), 16-byte
  * aligned; lengths a device int32 [batch]. head_dim 64 or 128, heads /
  * kv_heads <= 16. Split-K over positions: the split partials go to the
- * context's work buffer (allocated on first use, grown on demand). */
+ * context's work buffer (SH_ATTN_NOALLOC_MAX_BYTES on first use, grown by a
+ * call that needs more). */
 SH_API int sh_attn_decode_f16(sh_ctx *ctx, const float *q, const uint16_t *k, const uint16_t *v,
                               const int32_t *lengths, float *out, int batch, int heads,
                               int kv_heads, int head_dim, int max_positions, float scale);

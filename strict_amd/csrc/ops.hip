@@ -1095,7 +1095,10 @@ SH_API int sh_attn_decode_f16(sh_ctx *ctx, const float *q, const uint16_t *k, co
   int splits = 0, chunk = 0;
   attn_split(batch, heads, kv_heads, head_dim, max_positions, &splits, &chunk);
   void *part = nullptr;
-  if ((rc = context_scratch(ctx, attn_part_bytes(batch, heads, head_dim, splits), &part))) return rc;
+  // at least what the fine layout may ask for: a later call whose splits are finer
+  // finds its partials there and does not allocate (its stream may be capturing)
+  const size_t need = attn_part_bytes(batch, heads, head_dim, splits);
+  if ((rc = context_scratch(ctx, std::max(need, SH_ATTN_NOALLOC_MAX_BYTES), &part))) return rc;
   return run_attn(ctx, q, k, v, lengths, out, batch, heads, kv_heads, head_dim, max_positions, scale,
                   static_cast<float *>(part), splits, chunk);
 }
