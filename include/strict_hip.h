@@ -389,6 +389,14 @@ SH_API int sh_gemm_fp8(sh_ctx *ctx, const uint8_t *A, const float *sa, const uin
                        const float *sb, uint16_t *C, int M, int N, int K, int lda, int ldb,
                        int ldc);
 
+/* 1 where a call with these operands takes the 256 x 256 tiles, else 0 (for
+ * tests of that kernel; nothing is read or launched). */
+SH_API int sh_gemm_bf16_takes_256_tiles(const uint16_t *A, const uint16_t *B, const uint16_t *C,
+                                        int M, int N, int K, int lda, int ldb, int ldc);
+SH_API int sh_gemm_fp8_takes_256_tiles(const uint8_t *A, const uint8_t *Bt, const float *sb,
+                                       const uint16_t *C, int M, int N, int K, int lda, int ldb,
+                                       int ldc);
+
 /* ---- weight quantization ------------------------------------------------------
  * No reference counterpart: BASELINE configs[4] fixes the format. */
 

@@ -738,4 +738,15 @@ SH_API int sh_gemm_fp8(sh_ctx *ctx, const uint8_t *A, const float *sa, const uin
                   "gemm_fp8");
 }
 
+SH_API int sh_gemm_bf16_takes_256_tiles(const uint16_t *A, const uint16_t *B, const uint16_t *C,
+                                        int M, int N, int K, int lda, int ldb, int ldc) {
+  return gemm_bf16_uses_mfma(M, N, K, lda, ldb, ldc, A, B, C) ? 1 : 0;
+}
+
+SH_API int sh_gemm_fp8_takes_256_tiles(const uint8_t *A, const uint8_t *Bt, const float *sb,
+                                       const uint16_t *C, int M, int N, int K, int lda, int ldb,
+                                       int ldc) {
+  return gemm_fp8_uses_mfma(M, N, K, lda, ldb, ldc, A, Bt, C, sb) ? 1 : 0;
+}
+
 }  // extern "C"

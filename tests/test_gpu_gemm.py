@@ -13,6 +13,8 @@ import pytest
 
 import oracle
 import strict_amd
+from test_gpu_gemm_edge import _c, _place, _result
+from test_gpu_gemm_edge import _check as _check_bound
 
 pytestmark = pytest.mark.gpu
 
@@ -59,6 +61,45 @@ def test_gemm_4096_config(ctx):
     print(f"gemm 4096^3 max err / max |C| = {rel:.3e}")
 
 
+# The 256 x 256 tiles beyond 4096^3, at the bound of the any-shape kernel's tests:
+# grids that are no multiple of 256 tiles (ungrouped order), a grouped one that is
+# not square, K of one stage up to more than the pipeline holds. pad: elements after
+# each row of A, B (NaN) and of C; offset: elements before each operand
+@pytest.mark.parametrize("pad_ab,pad_c,offset", [(0, 0, 0), (8, 4, 8), (24, 12, 0)])
+@pytest.mark.parametrize("tiles_m,tiles_n,k", [(11, 13, 32), (11, 13, 64), (13, 11, 96), (11, 13, 160),
+                                               (13, 11, 320), (8, 32, 32), (8, 32, 224), (1, 131, 64),
+                                               (131, 1, 128)])
+def test_gemm_256_tiles(ctx, tiles_m, tiles_n, k, pad_ab, pad_c, offset):
+    m, n, lda, ldb = 256 * tiles_m, 256 * tiles_n, k + pad_ab, 256 * tiles_n + pad_ab
+    a, b = _bf16_operands(m, n, k, seed=m + n + k)
+    ba, va = _place(ctx, a, lda, offset, np.uint16(0x7FC0))
+    bb, vb = _place(ctx, b, ldb, offset, np.uint16(0x7FC0))
+    bc, vc = _c(ctx, m, n, n + pad_c, offset)
+    assert ctx._l.sh_gemm_bf16_takes_256_tiles(va.ptr, vb.ptr, vc.ptr, m, n, k, lda, ldb, n + pad_c)
+    ctx.gemm_bf16(va, vb, vc, m, n, k, lda, ldb, n + pad_c)
+    ctx.sync()
+    _check_bound(_result(bc, m, n, n + pad_c, offset), oracle.bf16_to_f32(a), oracle.bf16_to_f32(b))
+    for x in (ba, bb, bc):
+        x.free()
+
+
+def test_gemm_256_tiles_rule(ctx):
+    # one tile fewer, a remainder, an odd row or a misaligned operand: not these tiles
+    def takes(a, b, c, m, n, k, lda, ldb, ldc):
+        return ctx._l.sh_gemm_bf16_takes_256_tiles(a, b, c, m, n, k, lda, ldb, ldc)
+    m, n, k = 256 * 11, 256 * 12, 64
+    assert takes(4096, 4096, 4096, m, n, k, k, n, n) == 1
+    assert takes(4096, 4096, 4096, 256 * 8, 256 * 16, k, k, 256 * 16, 256 * 16) == 0
+    assert takes(4096, 4096, 4096, m, n, 48, 48, n, n) == 0
+    assert takes(4096, 4096, 4096, m - 1, n, k, k, n, n) == 0
+    assert takes(4096, 4096, 4096, m, n, k, k + 4, n, n) == 0
+    assert takes(4096, 4096, 4096, m, n, k, k, n + 4, n) == 0
+    assert takes(4096, 4096, 4096, m, n, k, k, n, n + 2) == 0
+    assert takes(4104, 4096, 4096, m, n, k, k, n, n) == 0
+    assert takes(4096, 4096, 4100, m, n, k, k, n, n) == 0
+
+
+# (too few tiles for the 256 x 256 ones: the any-shape kernel at multiples of its tiles)
 @pytest.mark.parametrize("m,n,k", [(256, 256, 64), (512, 768, 320), (768, 512, 4096),
                                    (1024, 2048, 128), (256, 512, 32), (512, 256, 96),
                                    (256, 256, 160)])

@@ -13,6 +13,7 @@ import pytest
 
 import oracle
 import strict_amd
+from test_gpu_gemm_edge import _c, _place, _result
 
 pytestmark = pytest.mark.gpu
 
@@ -61,6 +62,42 @@ def test_gemm_fp8_4096_config(ctx):
     print(f"gemm_fp8 4096^3 max err / max |C| = {rel:.3e}")
 
 
+# The 256 x 256 tiles beyond 4096^3, as in test_gpu_gemm.py, at this file's bar (the
+# scaled MFMA of these tiles does not sum a k-step's products in fp32: measured up to
+# 2^-16.5 of the sum of their magnitudes at K = 128, more than the any-shape kernel)
+@pytest.mark.parametrize("pad_ab,pad_c,offset", [(0, 0, 0), (16, 4, 16), (48, 12, 0)])
+@pytest.mark.parametrize("tiles_m,tiles_n,k", [(9, 11, 128), (11, 9, 256), (9, 11, 384), (11, 13, 640),
+                                               (8, 32, 128), (8, 32, 384), (1, 97, 256), (97, 1, 128)])
+def test_gemm_fp8_256_tiles(ctx, tiles_m, tiles_n, k, pad_ab, pad_c, offset):
+    m, n, ld = 256 * tiles_m, 256 * tiles_n, k + pad_ab
+    qa, sa, qb, sb = _operands(m, n, k, seed=m + n + k)
+    ba, va = _place(ctx, qa, ld, offset, np.uint8(0x7F))
+    bb, vb = _place(ctx, qb, ld, offset, np.uint8(0x7F))
+    bc, vc = _c(ctx, m, n, n + pad_c, offset)
+    dsa, dsb = ctx.upload(sa), ctx.upload(sb)
+    assert ctx._l.sh_gemm_fp8_takes_256_tiles(va.ptr, vb.ptr, dsb.ptr, vc.ptr, m, n, k, ld, ld, n + pad_c)
+    ctx.gemm_fp8(va, dsa, vb, dsb, vc, m, n, k, ld, ld, n + pad_c)
+    ctx.sync()
+    _check(_result(bc, m, n, n + pad_c, offset), _reference(qa, sa, qb, sb))
+    for x in (ba, bb, bc, dsa, dsb):
+        x.free()
+
+
+def test_gemm_fp8_256_tiles_rule(ctx):
+    def takes(a, b, s, c, m, n, k, lda, ldb, ldc):
+        return ctx._l.sh_gemm_fp8_takes_256_tiles(a, b, s, c, m, n, k, lda, ldb, ldc)
+    m, n, k = 256 * 9, 256 * 11, 256
+    assert takes(4096, 4096, 4096, 4096, m, n, k, k, k, n) == 1
+    assert takes(4096, 4096, 4096, 4096, 256 * 8, 256 * 12, k, k, k, 256 * 12) == 0
+    assert takes(4096, 4096, 4096, 4096, m, n, 192, 192, 192, n) == 0
+    assert takes(4096, 4096, 4096, 4096, m, n + 1, k, k, k, n + 3) == 0
+    assert takes(4096, 4096, 4096, 4096, m, n, k, k + 8, k, n) == 0
+    assert takes(4096, 4096, 4096, 4096, m, n, k, k, k, n + 2) == 0
+    assert takes(4104, 4096, 4096, 4096, m, n, k, k, k, n) == 0
+    assert takes(4096, 4096, 4100, 4096, m, n, k, k, k, n) == 0
+
+
+# (too few tiles for the 256 x 256 ones: the any-shape kernel at multiples of its tiles)
 @pytest.mark.parametrize("m,n,k", [(256, 256, 128), (512, 768, 384), (768, 512, 4096),
                                    (1024, 2048, 256)])
 def test_gemm_fp8_mfma_shapes(ctx, m, n, k):
