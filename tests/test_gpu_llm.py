@@ -223,6 +223,20 @@ def test_qwen3_small_head_as_separate_kernels(ctx, monkeypatch):
         _greedy_check(m, prompt, 64, "qwen3-small-head-separate")
 
 
+def _feed(m, prompts, steps, by_steps):
+    """Greedy tokens [batch, steps] after the prompts; by_steps: the prompts token by
+    token, logits-free but for the last, else in sh_llm_generate's one pass."""
+    if not by_steps:
+        return m.generate(prompts, steps)
+    for i in range(prompts.shape[1]):
+        m.step(prompts[:, i], logits=(i == prompts.shape[1] - 1))
+    toks = [m.next_tokens()]
+    for _ in range(steps - 1):
+        m.step(None, logits=True)
+        toks.append(m.next_tokens())
+    return np.stack(toks, axis=1)
+
+
 def test_qwen3_small_cooperative_launch(ctx, monkeypatch):
     # STRICT_HIP_LLM_COOP=1: the decode-layers kernel goes through HIP's
     # cooperative launch (residency guaranteed)
@@ -235,11 +249,13 @@ def test_qwen3_small_cooperative_launch(ctx, monkeypatch):
         _greedy_check(m, prompt, 64, "qwen3-small-coop")
 
 
+@pytest.mark.parametrize("by_steps", [True, False], ids=["steps", "generate"])
 @pytest.mark.parametrize("cfg", [QWEN_SMALL, GPT2_SMALL_TEST], ids=["qwen3", "gpt2"])
-def test_per_op_path_without_graphs(ctx, monkeypatch, cfg):
+def test_per_op_path_without_graphs(ctx, monkeypatch, cfg, by_steps):
     # STRICT_HIP_LLM_GRAPHS=0: the per-op path enqueues every kernel of a
-    # step eagerly instead of replaying its captured graph; tokens and
-    # logits equal the graph-replayed run's
+    # step eagerly instead of replaying its captured graphs (one with logits,
+    # one without: the prompt's steps); tokens and logits equal the
+    # graph-replayed run's
     monkeypatch.setenv("STRICT_HIP_LLM_LAYERS", "0")
     prompt = np.random.default_rng(21).integers(0, cfg.vocab, 10)
     runs = []
@@ -248,7 +264,7 @@ def test_per_op_path_without_graphs(ctx, monkeypatch, cfg):
         with llm.Model(ctx, cfg) as m:
             m.init_random(seed=9, stddev=0.02)
             m.reset(1)
-            toks = m.generate(prompt[None, :], 24)[0]
+            toks = _feed(m, prompt[None, :], 24, by_steps)[0]
             runs.append((toks, m.logits()[0].copy()))
     assert np.array_equal(runs[0][0], runs[1][0])
     assert np.array_equal(runs[0][1], runs[1][1])
@@ -638,23 +654,28 @@ def test_gpt2_xcd_local_placement_bit_identical(ctx, monkeypatch, cfg):
     assert np.array_equal(runs[0][1], runs[1][1])
 
 
-def test_gpt2_key_sets_across_batch_sizes(ctx):
+@pytest.mark.parametrize("by_steps", [True, False], ids=["steps", "generate"])
+def test_gpt2_key_sets_across_batch_sizes(ctx, by_steps):
     # GPT-2 runs its layers kernel at batch 1 (one launch per step, which
     # embeds the token itself and advances the step number, alternating the
-    # two argmax key sets) and the per-op path, graph-replayed, at batch 2.
-    # Between the two rounds' batch-2 runs, 15 + 16 = 31 layers-kernel steps
-    # move the current key set; each run must repeat the first round's tokens
-    # (a graph replayed on the other key set would not), and the history
-    # must hold the prompt and the generated tokens.
+    # two argmax key sets) and the per-op path, graph-replayed, at batch 2
+    # (the graph without logits too where the prompts go by steps). Between
+    # the two rounds' batch-2 runs, 15 + 16 = 31 layers-kernel steps (6 + 7 =
+    # 13 where all but a prompt's last token go in one pass) move the current
+    # key set; each run must repeat the first round's tokens (a graph replayed
+    # on the other key set would not), and the history must hold the prompt
+    # and the generated tokens.
     prompts = np.random.default_rng(31).integers(0, GPT2_SMALL_TEST.vocab, (2, 10))
     plan = ((1, 7), (2, 6), (1, 6))
+    moved = sum((10 if by_steps else 1) + steps - 1 for b, steps in plan if b == 1)
+    assert moved % 2 == 1  # an even number would end on the same key set
     with llm.Model(ctx, GPT2_SMALL_TEST) as m:
         m.init_random(seed=3, stddev=0.02)
         first = {}
         for rnd in range(2):
             for b, steps in plan:
                 m.reset(b)
-                toks = m.generate(prompts[:b], steps)
+                toks = _feed(m, prompts[:b], steps, by_steps)
                 print(f"round {rnd} batch {b} steps {steps}: {toks[0][:6]}", flush=True)
                 if rnd == 0:
                     first[(b, steps)] = toks
