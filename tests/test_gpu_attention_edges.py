@@ -77,3 +77,19 @@ def test_one_key_dominates(ctx):
     q, k, v, n = _inputs(4, 2, 16, 8, 128, 700, [700, 130])
     k[:, :, 129] = 6.0 * np.sign(q.reshape(2, 8, 2, 128)[:, :, 0]).astype(np.float16)
     _check(_run(ctx, q, k, v, n, 1.0), q, k, v, n, 1.0)
+
+
+# Calls whose splits of one tile would need over SH_ATTN_NOALLOC_MAX_BYTES of
+# partials or more than 1,024 splits: one split of 192 positions (a tile and a
+# half); 6 splits of 448; one of 192 (less than a tile of 256); 410 of 320
+@pytest.mark.parametrize("d,heads,kvh,batch,max_pos,lo", [(128, 16, 1, 2048, 130, 65), (128, 16, 1, 97, 2600, 1),
+                                                          (64, 16, 1, 4000, 130, 1), (128, 4, 1, 1, 131200, 131200)])
+def test_splits_that_are_no_multiple_of_a_tile(ctx, d, heads, kvh, batch, max_pos, lo):
+    tile = 128 if d == 128 else 256
+    tiles = -(-max_pos // tile)
+    fine = -(-tiles // max(1, -(-tiles * batch * kvh // 2048)))
+    assert fine > 1024 or batch * heads * fine * (d + 2) * 4 > 16 << 20
+    lens = np.random.default_rng(1).integers(lo, max_pos + 1, batch)
+    lens[0] = max_pos
+    q, k, v, n = _inputs(6, batch, heads, kvh, d, max_pos, lens)
+    _check(_run(ctx, q, k, v, n, 1 / np.sqrt(d)), q, k, v, n, 1 / np.sqrt(d))

@@ -102,3 +102,13 @@ def test_tallest_image(ctx, mode):
         assert np.array_equal(out.view(s + 2, n - 4).to_host(), ref[2:-2]) or s == h - n
     src.free()
     out.free()
+
+
+@pytest.mark.parametrize("delta,flags", [(40, 0), (40, 1), (-40, 0), (-40, 1), (0, 0)])
+def test_large_rgba_with_brightness(ctx, delta, flags):
+    # the RGBA streaming kernel with a partial last strip (2244 = 9 x 240 + 84
+    # pixels) and band (2237 = 139 x 16 + 13 rows), with and without alpha
+    w, h = 2244, 2237
+    img = seeded_bytes(w * h * 4, seed=delta + flags + 50)
+    got = _gpu(ctx, img, w, h, 4, strict_amd.BLUR_CONFIG, delta, flags)
+    assert np.array_equal(got, _reference(img, w, h, 4, strict_amd.BLUR_CONFIG, delta, bool(flags)))
