@@ -2,11 +2,13 @@
 (sh_llm_step, itself checked against the oracle in test_gpu_llm.py): KV
 caches of every layer, logits, lengths and history.
 
-Bounds: a K or V value is one fp16 rounding (2^-11) of a value whose inputs
-were rounded to fp16 twice per layer; the two paths sum in different orders, so
-some of those roundings flip by one step (2^-10). 4 x 2^-10 in the 2-norm and
-the attention bar of test_gpu_llm.py (1e-2 of the largest value) for the
-maximum hold both paths; a wrong position, head or mask is off by order 1."""
+The pass sums in the steps' own order and leaves their bits
+(test_gpu_prompt_exact.py). The bounds here are those of any order of sums: a
+K or V value is one fp16 rounding (2^-11) of a value whose inputs were rounded
+to fp16 twice per layer, and another order flips some of those roundings by one
+step (2^-10). 4 x 2^-10 in the 2-norm and the attention bar of test_gpu_llm.py
+(1e-2 of the largest value) for the maximum hold; a wrong position, head or
+mask is off by order 1."""
 import numpy as np
 import pytest
 
@@ -55,9 +57,8 @@ def _close(got, ref):
     assert np.max(np.abs(gl - rl)) <= LOGIT_REL_TOL * np.max(np.abs(rl))
 
 
-# 7: the fewest tokens that take the pass; 17, 65, 66: edges of the 16-token
-# q / k / v blocks and the 32- or 64-token attention blocks; 130, 301: a partial
-# last GEMM tile, several attention tiles
+# 7: less than a block; 17, 65, 66: edges of the 16-token q / k / v blocks and of
+# the 32-token GEMM tiles; 130, 301: a partial last tile, several splits
 @pytest.mark.parametrize("cfg,layers_kernel", [(QWEN_SMALL, "1"), (QWEN_SMALL, "0"),
                                                (QWEN_SMALL.with_(heads=2, hidden=512), "1"),
                                                (GPT2_SMALL_TEST, "1"),
@@ -102,9 +103,8 @@ def test_prompt_pass_after_cached_tokens(ctx, cfg):
             _close(_state(m, 2, total), ref)
 
 
-# the attention's blocks of 32 (head_dim 64: 64) tokens and tiles of 128 (64)
-# positions in four (two) parts: one token past a block, an odd and an even
-# number of blocks, one position past a part and past a tile
+# two tokens past 16-token blocks, an odd and an even number of 32-token blocks,
+# one and two positions past a 128-position part and past two
 @pytest.mark.parametrize("cfg", [QWEN_SMALL, GPT2_SMALL_TEST], ids=["qwen3", "gpt2"])
 @pytest.mark.parametrize("batch,n", [(2, 34), (1, 97), (1, 130), (2, 162), (1, 258)])
 def test_prompt_attention_block_edges(ctx, cfg, batch, n):
