@@ -18,7 +18,7 @@
 //    two stages ahead into a double-buffered LDS.
 // The element sums run in an order that depends on K and kGroups only.
 // It took the place of a bounds-checked fp32 FMA kernel: bf16 1000 x 1003 x 517
-// 78.3 -> 8.4 us, fp8 517 x 6144 x 1024 193 -> 16.4 us, bf16 4000 x 4001 x 3999
+// 78.3 -> 8.0 us, fp8 517 x 6144 x 1024 193 -> 15.5 us, bf16 4000 x 4001 x 3999
 // 213 us (0.60 PFLOP/s).
 //
 // Loads are 16 bytes at any element alignment. A chunk that crosses the end

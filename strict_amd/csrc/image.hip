@@ -406,7 +406,7 @@ __global__ __launch_bounds__(kBlock) void rgb_to_bgr_kernel(const uint8_t *__res
 // hold the clamped columns and pick them with v_perm; in reference mode the
 // outside bytes are then zeroed.
 // It took the place of one thread per pixel reading 25 taps of each channel
-// through the cache: 1919 x 1079 x 3 in reference mode 78.5 -> 7.0 us, 4096 x
+// through the cache: 1919 x 1079 x 3 in reference mode 78.5 -> 6.6 us, 4096 x
 // 4096 x 3 20 us (5.0 TB/s). Bound by vector instructions (about 75 per 8 bytes
 // and row) and, below some 2 million pixels, by one round of load latency.
 // ---------------------------------------------------------------------------
@@ -710,7 +710,7 @@ void launch_blur_bytes(hipStream_t s, const BytesArgs &a) {
 template <int kC>
 void launch_blur_channels(hipStream_t s, BytesArgs a, int mode) {
   a.strips = (int)((a.row_bytes + kStripBytes - 1) / kStripBytes);
-  // 4 rows per wave keep the chip full at ordinary sizes (1919 x 1079 x 3: 7.0 us
+  // 4 rows per wave keep the chip full at ordinary sizes (1919 x 1079 x 3: 6.6 us
   // against 8.6 with 8 rows); where there are waves enough, 8 rows re-read
   // fewer (4095 x 4095 x 4: 25.3 against 28.8)
   const long long waves8 = (long long)a.strips * ((a.height + 7) / 8);

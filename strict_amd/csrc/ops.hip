@@ -576,11 +576,13 @@ __device__ __forceinline__ void attn_fp32(const AttnOpArgs &a, int b, int kvh, i
 // 4.1e-7.)
 // Infinities do not survive that (a part of the other sign, or 0, times one is
 // NaN): a split whose sums are not finite is worked out again in fp32.
-// Measured, both kernels of a call, before and after: 4 rows up to 4,096
-// positions, 16 / 8 heads of 128: 29.7 -> 13.5 us (50 MB, 3.7 TB/s); 16 rows 68.3
-// -> 38.5 (4.7 TB/s); 16 rows of 8,192, 16 / 1 heads 73.7 -> 25.2; 1 row of 384,
-// 12 / 12 heads of 64 9.0 -> 8.2. fp32 FMAs from registers in its place were as
+// Measured, both kernels of a call, the fp32 kernel and this one: 4 rows of 4,096
+// positions, 16 / 8 heads of 128: 30.8 and 17.6 us (67 MB, 3.8 TB/s); 16 rows 72.4
+// and 49.3 (5.4 TB/s); 16 rows of 8,192, 16 / 1 heads 74.5 and 27.4; 1 row of 384,
+// 12 / 12 heads of 64 9.2 and 8.8. fp32 FMAs from registers in its place were as
 // fast at one query head per KV head and slower from two on (16 / 1 heads: 65.8).
+// (The low part's own sums cost 0.1 to 2.5 us of these; at head_dim 128, 7 values
+// beyond the 168 registers lie in scratch, 4 without those sums.)
 template <int kD>
 __global__ __launch_bounds__(kT, 3) void attn_op_partials_kernel(const AttnOpArgs a) {
   constexpr int kKK = kD / 32, kDT = kD / 16;
@@ -877,9 +879,13 @@ __global__ __launch_bounds__(kD * kMergeParts) void attn_op_merge_kernel(const A
 
 // Split layout of a call. The lengths are on the device, so the splits cover
 // max_pos; one of no active position ends at once. Splits of one tile, up to
-// about 2,048 workgroups (all resident together), of more tiles beyond that;
-// where the partials of that layout would exceed the allocation-free entry's
-// array, the coarser one of about two workgroups per CU.
+// about 2,048 workgroups, of more tiles beyond that. Three per CU, 768, are
+// resident together (registers; 42 KiB of LDS at head_dim 128), but planned for 768
+// a call took longer: 4 rows of 4,096 positions, 16 / 8 heads of 128, 19.0 us
+// against 17.5, 64 rows of 1,000 55.1 against 51.0, 1 row of 131,200, 4 / 1 heads,
+// a half-filled cache 25.3 against 20.3 (16 rows of 8,192, 16 / 1 heads 24.0
+// against 27.4); 1,536 is level. Where the partials of that layout would exceed the
+// allocation-free entry's array, the coarser one of about two workgroups per CU.
 void attn_split(int batch, int heads, int kv_heads, int head_dim, int max_pos, int *splits, int *chunk) {
   const long long rows = (long long)batch * kv_heads;
   const int tile = head_dim == 64 ? kAttnTile<64> : kAttnTile<128>;
