@@ -3,10 +3,9 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload decode|image|sigmoid]
 
-BASELINE.json's metric is "HBM GB/s (% peak) per kernel; decode tokens/s
-Qwen3-0.6B-shape FP8 b=1". The headline line (workload "decode") is
-configs[4] at batch 1: a Qwen3-0.6B-shaped decoder with random FP8-E4M3
-weights (per-output-channel fp32 scales), fp16 activations, a 4096-token KV
+The metric is "HBM GB/s (% peak) per kernel; decode tokens/s Qwen3-0.6B-shape
+FP8 b=1". The headline line (workload "decode") is a Qwen3-0.6B-shaped decoder
+at batch 1 with random FP8-E4M3 weights (per-output-channel fp32 scales), fp16 activations, a 4096-token KV
 cache filled by a 4096-token random prompt, then K greedy decode steps timed
 (a "step" = one token for every sequence). Its roofline is the step's
 algorithmic bytes (weights + scales + norms + K/V of every cached position)
@@ -15,9 +14,9 @@ over the measured step time, against 8 TB/s.
 Every other kernel of the path is timed the same way and listed under
 "kernels" with its algorithmic GB/s (or TFLOP/s) and fraction of peak:
 copy (HBM calibration), brightness, 5x5 blur, the fused brightness+blur of
-configs[1], the unfused pipeline, sigmoid, the bf16 GEMM
-(configs[2]), the FP8 GEMV at the LM-head shape, Qwen3 decode at b=4 and
-b=16, GPT-2 (configs[3]) decode.
+a 4096 x 4096 image, the unfused pipeline, sigmoid over 2^24 values, the bf16
+GEMM, the FP8 GEMV at the LM-head shape, Qwen3 decode at b=4 and
+b=16, GPT-2 small decode.
 
 Every row carries a cpu_baseline timed on this host after the GPU work: the
 reference's own CPU code restated in C (oracle/oracle.c) in TestPerformance's
@@ -386,7 +385,7 @@ def decode_run(ctx, cfg, batch, prompt_len, steps, warmup, seed=42):
 # ---- CPU baselines (the oracle, timed on this host) ------------------------
 
 def cpu_baseline_decode(seconds: float):
-    """numpy oracle of the Qwen3 configs[4] decode step at b = 1 on a 4096-token
+    """numpy oracle of the Qwen3 decode step at b = 1 on a 4096-token
     KV cache (random fp32 weights of the config's shapes, random K/V)."""
     import oracle.llm as ollm
     from strict_amd import llm
@@ -667,7 +666,7 @@ def cpu_baseline_gemv():
 
 
 def cpu_baseline_gpt2(seconds: float):
-    """numpy oracle of the GPT-2 configs[3] decode step at b=1 after a 128-token prompt."""
+    """numpy oracle of the GPT-2 decode step at b=1 after a 128-token prompt."""
     import oracle.llm as ollm
     from strict_amd import llm
 

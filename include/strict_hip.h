@@ -365,7 +365,7 @@ SH_API int sh_rgb_to_bgr_u8(sh_ctx *ctx, const uint8_t *src, uint8_t *dst, int w
 
 /* ---- typed ops: dense GEMM --------------------------------------------------
  * The reference's only GEMM hook is the cuBLAS handle of Kernel.Handle
- * (Kernel.cs:10-11, :16), never used; BASELINE configs[2] fixes the op. */
+ * (Kernel.cs:10-11, :16), never used. */
 
 /* C[M,N] = A[M,K] * B[K,N]: bf16 operands (raw 16-bit patterns), fp32
  * accumulation, bf16 result (round to nearest even), row-major with leading
@@ -398,7 +398,7 @@ SH_API int sh_gemm_fp8_takes_256_tiles(const uint8_t *A, const uint8_t *Bt, cons
                                        int ldc);
 
 /* ---- weight quantization ------------------------------------------------------
- * No reference counterpart: BASELINE configs[4] fixes the format. */
+ * No reference counterpart. */
 
 /* Per-row OCP E4M3 quantization of a device fp32 matrix W[N][K]:
  * scale[n] = max_k |W[n][k]| / 448 (1 for an all-zero row), q = e4m3(W / scale)
@@ -476,9 +476,9 @@ SH_API int sh_attn_decode_f16_noalloc(sh_ctx *ctx, const float *q, const uint16_
                                       int max_positions, float scale);
 
 /* ---- LLM decode (model runners) ------------------------------------------------
- * No reference counterpart: BASELINE configs[3] (GPT-2 small, fp16 weights)
- * and configs[4] (Qwen3-0.6B shape, FP8-E4M3 weights with per-output-channel
- * fp32 scales) define the models. One sh_llm owns its weights, KV cache and
+ * No reference counterpart. The models: GPT-2 (measured as GPT-2 small, fp16
+ * weights) and Qwen3 (the 0.6B shape, FP8-E4M3 weights with per-output-channel
+ * fp32 scales). One sh_llm owns its weights, KV cache and
  * work buffers on the context's device; steps are ordered on the context's
  * stream and replayed from a HIP graph after the first step of a batch. */
 

@@ -1,16 +1,15 @@
 """CPU oracle of the LLM decode path -- TEST INFRASTRUCTURE ONLY.
 
 The reference (strict-lang/Strict) has no LLM, GEMM, FP8, attention or norm
-code at all (SURVEY rows a13-a16 are defined by BASELINE.json configs[3] and
-configs[4] alone), so this module restates the two model definitions from
+code at all, so this module restates the two model definitions from
 their published architectures in numpy:
 
-- Qwen3 (configs[4]): RMSNorm (eps 1e-6) -> fused QKV projection -> per-head
+- Qwen3: RMSNorm (eps 1e-6) -> fused QKV projection -> per-head
   RMSNorm of q and k -> RoPE rotate-half (theta 1e6) -> GQA softmax attention
   -> O projection + residual -> RMSNorm -> SwiGLU MLP + residual; final
   RMSNorm; LM head tied to the token embedding. Linear weights are OCP E4M3
   with one fp32 scale per output row.
-- GPT-2 (configs[3]): token + learned position embedding -> LayerNorm (eps
+- GPT-2: token + learned position embedding -> LayerNorm (eps
   1e-5) -> QKV (+bias) -> MHA -> O (+bias) + residual -> LayerNorm -> GELU
   (tanh) MLP (+biases) + residual; final LayerNorm; LM head tied to wte.
   Weights fp16.

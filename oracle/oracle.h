@@ -51,8 +51,8 @@ void or_adjust_brightness(const uint8_t *in, uint8_t *out, size_t pixels, int ch
 void or_blur5_reference(const uint8_t *in, uint8_t *out, int width, int height, int channels,
                         int nthreads);
 
-/* Config semantics (no reference implementation; fixed by BASELINE.json
- * configs[1]): 5x5 box, clamp-to-edge coordinates, (sum + 12) / 25. */
+/* Config semantics (no reference implementation): 5x5 box, clamp-to-edge
+ * coordinates, (sum + 12) / 25. */
 void or_blur5_config(const uint8_t *in, uint8_t *out, int width, int height, int channels,
                      int nthreads);
 

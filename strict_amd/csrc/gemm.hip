@@ -1,6 +1,6 @@
 // Dense GEMM C[M,N] = A[M,K] * B[K,N], bf16 operands, fp32 accumulation,
 // bf16 output, all row-major. The reference only holds an unused cuBLAS
-// handle for this (Kernel.cs:10-11, :16); the workload is BASELINE configs[2].
+// handle for this (Kernel.cs:10-11, :16); the measured shape is 4096^3.
 //
 // MFMA kernel (M % 256 == 0, N % 256 == 0, K % 32 == 0, leading dimensions
 // multiples of 8 elements, 16-byte aligned operands):

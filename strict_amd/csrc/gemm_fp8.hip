@@ -3,8 +3,7 @@
 // row-major (each output column's K values contiguous, the layout of a
 // weight matrix W[N][K] quantized per output row); sa / sb are the fp32
 // per-row / per-column scales (sh_quantize_e4m3 makes both). OCP E4M3.
-// The reference has nothing for this (BASELINE's FP8 GEMM
-// measurement); the decode path's prefill shape is M = 4096 tokens.
+// The reference has nothing for this; the measured shape is 4096^3.
 //
 // MFMA kernel (M % 256 == 0, N % 256 == 0, K % 128 == 0, leading dimensions
 // multiples of 16 bytes, 16-byte aligned A / Bt, 8-byte aligned C):

@@ -1,8 +1,7 @@
-// Kernels of the LLM decode path (BASELINE configs[3] GPT-2 small fp16 and
-// configs[4] Qwen3-0.6B-shaped FP8): weight quantization / tiling, a fused
+// Kernels of the LLM decode path (GPT-2 small fp16 and
+// Qwen3-0.6B-shaped FP8): weight quantization / tiling, a fused
 // batched GEMV on MFMA, split-K decode attention and the embedding gather.
-// The reference has no implementation of any of these (SURVEY rows a14-a16
-// of the hot path are defined by BASELINE.json only).
+// The reference has no implementation of any of these.
 //
 // Weight layout ("tiled"): a linear layer W[N][K] (N outputs, K inputs) is
 // stored as 1 KiB tiles of 16 rows, tiles of one row group consecutive along

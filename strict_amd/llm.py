@@ -1,7 +1,7 @@
-"""Greedy decoding of the BASELINE LLM configs through libstrict_hip's sh_llm_*
+"""Greedy decoding of the two LLM workloads through libstrict_hip's sh_llm_*
 C ABI: GPT-2 small (fp16 weights) and the Qwen3-0.6B shape (FP8-E4M3
 weights with per-output-channel fp32 scales). The reference has no LLM path
-at all; the configs in BASELINE.json define these models.
+at all; the models are their published architectures at these sizes.
 
 Weights are random (``init_random``: N(0, stddev) from a counter-based
 generator on the device) or loaded per linear from fp32 arrays
@@ -47,11 +47,11 @@ class Config:
         return (self.vocab + 15) // 16 * 16
 
 
-# BASELINE configs[4]: Qwen3-0.6B shape, 4096-token KV cache (+ 256 decode steps)
+# Qwen3-0.6B shape, 4096-token KV cache (+ 256 decode steps)
 QWEN3_0_6B = Config(QWEN3, layers=28, hidden=1024, heads=16, kv_heads=8, head_dim=128,
                     intermediate=3072, vocab=151936, max_positions=4096 + 256,
                     rope_theta=1e6, norm_eps=1e-6)
-# BASELINE configs[3]: GPT-2 small, ctx 1024
+# GPT-2 small, ctx 1024
 GPT2_SMALL = Config(GPT2, layers=12, hidden=768, heads=12, kv_heads=12, head_dim=64,
                     intermediate=3072, vocab=50257, max_positions=1024, norm_eps=1e-5)
 

@@ -52,7 +52,7 @@ def declared_arities():
 
 
 def csharp_bindings():
-    """name -> parameter count of every `static extern` in INTEGRATION.md's C# blocks."""
+    """name -> parameter count of every `static extern` in the integration guide's C# blocks."""
     text = (ROOT / "INTEGRATION.md").read_text()
     out = {}
     for block in re.findall(r"```csharp\n(.*?)```", text, re.S):
@@ -63,7 +63,7 @@ def csharp_bindings():
 
 
 def test_csharp_binding_covers_every_symbol():
-    # the P/Invoke layer a C# host adds declares every
+    # the P/Invoke layer a C# host adds (the integration guide) declares every
     # export of include/*.h, with the header's parameter count
     declared, bound = declared_arities(), csharp_bindings()
     assert set(declared) == set(declared_symbols())

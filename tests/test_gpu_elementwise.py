@@ -9,7 +9,7 @@ from tests.util import seeded_uniform_f32, ulp_distance_f32
 
 pytestmark = pytest.mark.gpu
 
-N_CONFIG = 1 << 24
+N_CONFIG = 1 << 24  # the measured sigmoid workload
 
 
 def _run_sigmoid(ctx, x):
@@ -24,13 +24,13 @@ def _run_sigmoid(ctx, x):
 
 
 def test_sigmoid_config_2pow24_within_2ulp(ctx):
-    # configs[0]: N = 2^24 values uniform[-8, 8] from a seeded generator
+    # N = 2^24 values uniform[-8, 8] from a seeded generator
     x = seeded_uniform_f32(N_CONFIG, -8.0, 8.0, seed=42)
     y = _run_sigmoid(ctx, x)
     ref = oracle.sigmoid_f32(x, nthreads=oracle.default_threads())
     d = ulp_distance_f32(y, ref)
     print(f"sigmoid 2^24: max ulp {d.max()}, bit-exact {np.mean(d == 0):.4f}", flush=True)
-    assert d.max() <= 2  # north_star: sigmoid within 2 ulp fp32
+    assert d.max() <= 2  # sigmoid within 2 ulp fp32
 
 
 def test_sigmoid_special_values_and_tails(ctx):

@@ -2,8 +2,8 @@
 
 C[m,n] = sa[m] * sb[n] * sum_k e4m3(A[m,k]) * e4m3(Bt[n,k]), fp32 accumulation,
 bf16 output; A and Bt quantized per row (oracle.quantize_e4m3_rows, the same
-rule as sh_quantize_e4m3). The reference has no GEMM; BASELINE's FP8 GEMM
-measurement fixes 4096^3 with per-row / per-column scales. Reference product:
+rule as sh_quantize_e4m3). The reference has no GEMM; the measured
+workload is 4096^3 with per-row / per-column scales. Reference product:
 the dequantized operands multiplied with double accumulation (oracle.gemm_f32).
 Tolerance, as for the bf16 GEMM:
   max |C_gpu - C_ref| <= 1e-2 * max |C_ref|  and  ||C_gpu - C_ref|| <= 1e-2 ||C_ref||.

@@ -9,7 +9,7 @@ from tests.util import seeded_bytes
 
 pytestmark = pytest.mark.gpu
 
-W = H = 4096
+W = H = 4096  # the measured image workload
 NT = oracle.default_threads()
 
 

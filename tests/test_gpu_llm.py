@@ -1,10 +1,10 @@
 """GPU parity of the LLM decode path (FP8 quantizer, W8A16 GEMV, GPT-2 and
 Qwen3-shaped greedy decoding) against the numpy oracle (oracle/llm.py).
 
-The reference has no implementation of any of these
-(GPT-2 small, fp16, 128-token prompt, 256 greedy steps) and configs[4]
-(Qwen3-0.6B shape, FP8 weights, fp16 activations) define them. North-star
-bar: identical greedy top-1 tokens, with the logit max-abs-diff stated.
+The reference has no implementation of any of these; the workloads are
+GPT-2 small (fp16, 128-token prompt, 256 greedy steps) and the Qwen3-0.6B
+shape (FP8 weights, fp16 activations). Bar: identical greedy
+top-1 tokens, with the logit max-abs-diff stated.
 
 Greedy comparison is teacher-forced: the oracle is fed the GPU's tokens and
 its own argmax is compared at every step. Tolerances (stated here):
@@ -15,7 +15,7 @@ its own argmax is compared at every step. Tolerances (stated here):
     margin is below twice the observed logit max-abs-diff (a tie at the
     precision both sides share) may pick either of the tied tokens; such
     steps are counted and printed;
-  - configs[3] (GPT-2, 256 steps): in addition, identical at every step,
+  - GPT-2 small (256 steps): in addition, identical at every step,
     near-ties included, to the oracle with its linears summed in fp64.
 """
 import numpy as np
@@ -315,7 +315,7 @@ def test_gpt2_full_width_three_and_four_splits(ctx):
     # GPT-2 small's widths with max_positions 160: 48-position attention
     # splits, so a 140-token prompt and 16 steps (contexts 141..156) run the
     # O items' staging over 3 and then 4 active splits per head at hidden
-    # 768 (two dim pairs per lane), which configs[3] (256-position splits)
+    # 768 (two dim pairs per lane), which GPT-2 small (256-position splits)
     # reaches only past 512 positions
     cfg = llm.GPT2_SMALL.with_(max_positions=160)
     with llm.Model(ctx, cfg) as m:
@@ -327,7 +327,7 @@ def test_gpt2_full_width_three_and_four_splits(ctx):
 
 
 def test_gpt2_config3_greedy_256(ctx):
-    # BASELINE configs[3]: GPT-2 small, random N(0, 0.02) fp16 weights, batch 1,
+    # GPT-2 small, random N(0, 0.02) fp16 weights, batch 1,
     # 128-token prompt of seeded uniform ids, 256 greedy steps with KV cache
     cfg = llm.GPT2_SMALL
     with llm.Model(ctx, cfg) as m:
@@ -340,16 +340,16 @@ def test_gpt2_config3_greedy_256(ctx):
         _greedy_check(m, prompt, 256, "gpt2-config3", exact64=True)
 
 
-# ---- configs[4] at its own shape: one model, max_batch 16, KV room for 4096+ --------
+# ---- the Qwen3-0.6B shape: one model, max_batch 16, KV room for 4096+ --------
 
 QWEN_CONFIG4 = llm.QWEN3_0_6B.with_(max_positions=4096 + 64, max_batch=16)
 
 
 @pytest.fixture(scope="module")
 def config4(ctx):
-    """The configs[4] model (28 layers, hidden 1024, 16 Q / 8 KV heads, head_dim
+    """The Qwen3-0.6B-shaped model (28 layers, hidden 1024, 16 Q / 8 KV heads, head_dim
     128, SwiGLU 3072, vocab 151936, FP8 weights) and its dequantized weights
-    for the oracle, shared by the configs[4] tests."""
+    for the oracle, shared by the tests of that shape."""
     m = llm.Model(ctx, QWEN_CONFIG4)
     m.init_random(seed=42, stddev=0.02)
     assert m.uses_layers_kernel
@@ -415,14 +415,14 @@ def _check_kv_cache(model, decs, label):
 
 
 def test_qwen3_config4_greedy_256(ctx, config4):
-    # BASELINE configs[4] at batch 1: 32-token prompt, 256 greedy steps
+    # the Qwen3-0.6B shape at batch 1: 32-token prompt, 256 greedy steps
     m, w = config4
     prompt = np.random.default_rng(42).integers(0, QWEN_CONFIG4.vocab, (1, 32))
     _batch_greedy_check(m, w, prompt, 256, "qwen3-config4-b1")
 
 
 def test_qwen3_config4_xcd_local_placement_bit_identical(ctx, config4, monkeypatch):
-    # Batch 1 at configs[4]'s shape runs XCD-local: KV head h's QKV tiles,
+    # Batch 1 at the Qwen3-0.6B shape runs XCD-local: KV head h's QKV tiles,
     # attention splits and merge items on XCD h, their cells stored into
     # that XCD's L2. The items and their arithmetic are the same as with the
     # default placement (STRICT_HIP_LLM_XCD=0), so logits and tokens of 24
@@ -452,7 +452,7 @@ def test_qwen3_config4_xcd_local_placement_bit_identical(ctx, config4, monkeypat
 
 @pytest.mark.parametrize("batch", [4, 6, 8, 16])
 def test_qwen3_config4_batch_vs_oracle(ctx, config4, batch):
-    # configs[4] at batch 4 to 16 after 12-token prompts: every row its own
+    # the Qwen3-0.6B shape at batch 4 to 16 after 12-token prompts: every row its own
     # prompt, each checked against its own oracle decoder, and every row's K
     # and V^T cache entries against the oracle's. At this length each (row,
     # KV head) has one active attention split, so every workgroup runs at
@@ -506,7 +506,7 @@ def _batch_long_check(model, weights, prompts, steps, single_rows, oracle_rows, 
           f"{worst:.3e}, token mismatches {ties} (all near-ties)")
 
 
-# Attention items at configs[4]'s split size (144 positions, 32 splits per
+# Attention items at the Qwen3-0.6B split size (144 positions, 32 splits per
 # (row, KV head)): a context of ~2,200 positions has 16 active splits per
 # (row, KV head), one of ~4,100 has 29. The 256 workgroups' runs then are:
 #   b = 4  (small-batch kernel, the active items partitioned by a cursor):
@@ -532,7 +532,7 @@ def test_qwen3_config4_batch_long_prompt_rows(ctx, config4, batch, rows):
 
 
 def test_qwen3_config4_batch4_kv4096(ctx, config4):
-    # BASELINE configs[4] at batch 4 against a 4096-token KV cache: every row
+    # the Qwen3-0.6B shape at batch 4 against a 4096-token KV cache: every row
     # against batch 1, row 0 against the oracle
     m, w = config4
     prompts = np.random.default_rng(11).integers(0, QWEN_CONFIG4.vocab, (4, 4096))
@@ -540,7 +540,7 @@ def test_qwen3_config4_batch4_kv4096(ctx, config4):
 
 
 def test_qwen3_config4_batch16_kv4096(ctx, config4):
-    # BASELINE configs[4] at batch 16 against a 4096-token KV cache: rows from
+    # the Qwen3-0.6B shape at batch 16 against a 4096-token KV cache: rows from
     # both staging passes of the GEMV items (0-7, 8-15) against batch 1, row
     # 15 against the oracle
     m, w = config4
@@ -549,7 +549,7 @@ def test_qwen3_config4_batch16_kv4096(ctx, config4):
 
 
 def test_qwen3_long_context_step(ctx, config4):
-    # BASELINE configs[4] KV length: a 4096-token prompt fills the cache, then
+    # the Qwen3-0.6B shape's KV length: a 4096-token prompt fills the cache, then
     # greedy steps attend over 4096+ positions (split-K attention with many
     # splits and the cross-workgroup merge)
     m, w = config4

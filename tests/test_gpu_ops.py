@@ -142,7 +142,7 @@ def test_argmax_vs_numpy(ctx):
 
 
 @pytest.mark.parametrize("batch,heads,kv_heads,d,max_pos,lengths", [
-    (1, 16, 8, 128, 4096, [4096]),                 # configs[4] shape, full cache
+    (1, 16, 8, 128, 4096, [4096]),                 # the Qwen3-0.6B shape, full cache
     (3, 16, 8, 128, 4133, [1, 4133, 2000]),        # ragged, a partial last tile
     (4, 12, 12, 64, 384, [384, 0, 129, 64]),       # GPT-2 MHA, an empty row
     (2, 16, 1, 128, 300, [300, 65]),               # 16 query heads on one KV head

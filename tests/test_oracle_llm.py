@@ -166,7 +166,7 @@ def test_inv_freq_matches_transformers_rope_init():
 
 
 def test_decode_step_bytes_config4():
-    # SURVEY 8(d): 598,099,456 B of weights + 469,762,048 B of KV at b = 1, 4096
+    # 598,099,456 B of weights + 469,762,048 B of KV at b = 1, 4096
     # positions; this build also counts norm gains of the q/k head norms and
     # the embedding row, so the weights figure is within 0.1 %
     b = llm.decode_step_bytes(llm.QWEN3_0_6B, 1, 4096)
