@@ -41,11 +41,6 @@ struct Layer {
   uint16_t *kcache = nullptr, *vcache = nullptr;
 };
 
-// Splits of the context per (sequence, KV head): about 512 workgroups in all
-// (two per CU; at the Qwen3 shape and b = 1, 64 splits of <= 80 positions up
-// to 5120 tokens, so each workgroup's K and V fit one batch of loads issued
-// together), at least enough that no split exceeds kMaxSplitChunk positions,
-// at most 64 (the merge kernel's limit).
 // Splits per (row, KV head) of the per-op attention kernel: as few as keep a
 // split within kMaxSplitChunk positions. Each kernel of a per-op step costs
 // ~4-6 us whatever its size (measured on GPT-2's step), so one split per
@@ -533,7 +528,8 @@ int prefill_slice(const sh_llm *m, int rows) {
 }
 
 // The parts of the work buffer for `rows` token rows, each at a multiple of
-// 256 bytes; returns the whole size (base NULL: only that).
+// 256 bytes; returns the whole size (base NULL: only that). Nothing in it depends
+// on the batch but through `rows`: a buffer kept from one batch serves another.
 size_t prefill_layout(const sh_llm *m, int rows, uint8_t *base, PrefillArgs *a, float **qkv,
                       uint16_t **act, float **partials) {
   const sh_llm_config &c = m->cfg;
