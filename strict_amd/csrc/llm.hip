@@ -944,6 +944,8 @@ SH_API int sh_llm_init_random(sh_llm *m, uint64_t seed, float stddev) {
   for (Layer &L : m->layers)
     for (Linear *l : {&L.qkv, &L.o, &L.up, &L.down})
       if ((size_t)l->N * l->K > max_elems) max_elems = (size_t)l->N * l->K;
+  // (the position table passes through it, too, and may be the largest)
+  if (m->wpe) max_elems = std::max(max_elems, (size_t)m->cfg.max_positions * m->cfg.hidden);
   float *tmp = nullptr;
   SH_HIP_TRY(hipMalloc(&tmp, max_elems * sizeof(float)));
   uint64_t stream_id = seed * 1000003ull;

@@ -686,6 +686,20 @@ def test_gpt2_key_sets_across_batch_sizes(ctx, by_steps):
                 assert np.array_equal(hist[10:], toks[0][:steps - 1])
 
 
+def test_init_random_with_a_position_table_larger_than_every_linear(ctx):
+    # 3,000 x 256 positions beside linears of at most 1,008 x 256: the table is
+    # random to its end, and the weights are those of a model with a small table
+    heads = []
+    for positions in (512, 3000):
+        with llm.Model(ctx, GPT2_SMALL_TEST.with_(max_positions=positions)) as m:
+            m.init_random(seed=3, stddev=0.02)
+            heads.append(m.read("head.w", 0).copy())
+            wpe = m.read("wpe", 0, np.float16).reshape(positions, -1).astype(np.float32)
+            for rows in (wpe[:100], wpe[-100:]):
+                assert abs(rows.std() - 0.02) < 0.002 and abs(rows.mean()) < 0.002
+    assert np.array_equal(heads[0], heads[1])
+
+
 def test_llm_rejects_bad_arguments(ctx):
     with pytest.raises(strict_amd.StrictHipError):
         llm.Model(ctx, QWEN_SMALL.with_(head_dim=96))
