@@ -50,7 +50,8 @@ def _check(m, batch, n, seed=3):
 #  - splits of 512 positions: four 128-position halves, the softmax sums' lanes
 #    taken a second time;
 #  - GPT-2 on its layers kernel (batch 1, splits of 256) and on the per-op
-#    kernels (other batches); the per-op kernels of Qwen3, one split and three
+#    kernels (other batches; one split and three); the per-op kernels of Qwen3, one
+#    split and three
 CASES = [
     ("qwen3-wide", QWEN_WIDE, "1", [(1, 5), (1, 145), (1, 290), (2, 161), (4, 67), (16, 21)]),
     ("qwen3-wide-long", QWEN_WIDE, "1", [(1, 2450)]),
@@ -64,6 +65,7 @@ CASES = [
     ("qwen3-per-op", QWEN_SMALL, "0", [(1, 7), (1, 130), (3, 65)]),
     ("qwen3-per-op-mha", QWEN_SMALL.with_(heads=2, hidden=512), "1", [(2, 66)]),
     ("qwen3-per-op-splits", QWEN_SMALL.with_(max_positions=2100), "0", [(2, 720)]),
+    ("gpt2-per-op-splits", GPT2_SMALL_TEST.with_(max_positions=2100), "1", [(1, 1060), (2, 66)]),
 ]
 
 
